@@ -93,11 +93,37 @@ template <typename R> __device__ __forceinline__ double s_mag(cx<R> a) {
 __device__ __forceinline__ float  s_magr(float a)  { return __builtin_fabsf(a); }
 __device__ __forceinline__ double s_magr(double a) { return __builtin_fabs(a); }
 template <typename R> __device__ __forceinline__ R s_magr(cx<R> a) { return s_magr(a.re) + s_magr(a.im); }
-// reciprocal of a pivot: FP32 takes the hardware reciprocal (1 ulp; FP32 factors only seed the
-// refinement), FP64 and complex the correctly rounded division
+// reciprocal of a pivot, on the serial chain of every inversion: FP32 takes the hardware reciprocal
+// (1 ulp; FP32 factors only seed the refinement), FP64 the hardware seed (better than 2^-24) and two
+// Newton steps r + r (1 - a r) in fused arithmetic, which end within an ulp: six dependent
+// instructions instead of the scaled division's eleven.  The seed's own value is kept where a step
+// would not be finite (zero, infinite or denormal pivots, as the division gives them).
 __device__ __forceinline__ float  s_recip_piv(float a)  { return __builtin_amdgcn_rcpf(a); }
-__device__ __forceinline__ double s_recip_piv(double a) { return 1.0 / a; }
-template <typename R> __device__ __forceinline__ cx<R> s_recip_piv(cx<R> a) { return s_recip(a); }
+__device__ __forceinline__ double s_recip_piv(double a) {
+    const double r0 = __builtin_amdgcn_rcp(a);
+    const double r1 = __builtin_fma(r0, __builtin_fma(-a, r0, 1.0), r0);
+    const double r2 = __builtin_fma(r1, __builtin_fma(-a, r1, 1.0), r1);
+    return __builtin_isfinite(r2) ? r2 : r0;
+}
+// complex: conj(a) / |a|^2 on a scaled to a larger part in [1/2, 1) (exponents moved exactly), without
+// the branch and the two divisions of s_recip
+__device__ __forceinline__ zf s_recip_piv(zf a) {
+    const int e = __builtin_amdgcn_frexp_expf(s_magr(a.re) > s_magr(a.im) ? a.re : a.im);
+    const float x = __builtin_ldexpf(a.re, -e), y = __builtin_ldexpf(a.im, -e);
+    const float r = s_recip_piv(x * x + y * y);
+    return {__builtin_ldexpf(x * r, -e), __builtin_ldexpf(-y * r, -e)};
+}
+__device__ __forceinline__ zd s_recip_piv(zd a) {
+    const int e = __builtin_amdgcn_frexp_exp(s_magr(a.re) > s_magr(a.im) ? a.re : a.im);
+    const double x = __builtin_ldexp(a.re, -e), y = __builtin_ldexp(a.im, -e);
+    const double r = s_recip_piv(x * x + y * y);
+    return {__builtin_ldexp(x * r, -e), __builtin_ldexp(-y * r, -e)};
+}
+// componentwise select (a conditional expression over complex values becomes a select of addresses,
+// which keeps the operands in scratch memory)
+__device__ __forceinline__ float  s_sel(bool c, float a, float b)   { return c ? a : b; }
+__device__ __forceinline__ double s_sel(bool c, double a, double b) { return c ? a : b; }
+template <typename R> __device__ __forceinline__ cx<R> s_sel(bool c, cx<R> a, cx<R> b) { return {c ? a.re : b.re, c ? a.im : b.im}; }
 __device__ __forceinline__ bool s_finite(float a)  { return __builtin_isfinite(a); }
 __device__ __forceinline__ bool s_finite(double a) { return __builtin_isfinite(a); }
 template <typename R> __device__ __forceinline__ bool s_finite(cx<R> a) { return __builtin_isfinite(a.re) && __builtin_isfinite(a.im); }
@@ -193,11 +219,58 @@ template <typename T, int N> __device__ __forceinline__ void tiles_settle(Tile<T
         asm volatile("s_nop 7\n\ts_nop 7" : "+a"(x[0].v), "+a"(x[1].v), "+a"(x[2].v));
     } else if constexpr (!tr<T>::C && N == 4) {
         asm volatile("s_nop 7\n\ts_nop 7" : "+a"(x[0].v), "+a"(x[1].v), "+a"(x[2].v), "+a"(x[3].v));
+    } else if constexpr (!tr<T>::C && N == 8) {
+        asm volatile("s_nop 7\n\ts_nop 7" : "+a"(x[0].v), "+a"(x[1].v), "+a"(x[2].v), "+a"(x[3].v), "+a"(x[4].v),
+                     "+a"(x[5].v), "+a"(x[6].v), "+a"(x[7].v));
     } else if constexpr (tr<T>::C && N == 2) {
         asm volatile("s_nop 7\n\ts_nop 7" : "+a"(x[0].re), "+a"(x[0].im), "+a"(x[1].re), "+a"(x[1].im));
+    } else if constexpr (tr<T>::C && N == 4) {
+        asm volatile("s_nop 7\n\ts_nop 7" : "+a"(x[0].re), "+a"(x[0].im), "+a"(x[1].re), "+a"(x[1].im), "+a"(x[2].re),
+                     "+a"(x[2].im), "+a"(x[3].re), "+a"(x[3].im));
     } else {
 #pragma unroll
         for (int i = 0; i < N; ++i) tile_settle(x[i]);
+    }
+#else
+    (void)x;
+#endif
+}
+
+// The same waits for accumulators kept in the vector registers.  Naming accumulation registers makes
+// the compiler split a kernel's registers between the two files, half and half where the launch
+// bounds limit them, and spill: the factor's tiles, which vector code and LDS writes read, stay in
+// the vector file (b = 128: 512 threads no longer held to 128 vector registers).
+template <typename T> __device__ __forceinline__ void tile_settle_v(Tile<T> &x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (tr<T>::C) {
+        asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x.re), "+v"(x.im));
+    } else {
+        asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x.v));
+    }
+#else
+    (void)x;
+#endif
+}
+
+template <typename T, int N> __device__ __forceinline__ void tiles_settle_v(Tile<T> (&x)[N]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (!tr<T>::C && N == 2) {
+        asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x[0].v), "+v"(x[1].v));
+    } else if constexpr (!tr<T>::C && N == 3) {
+        asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x[0].v), "+v"(x[1].v), "+v"(x[2].v));
+    } else if constexpr (!tr<T>::C && N == 4) {
+        asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x[0].v), "+v"(x[1].v), "+v"(x[2].v), "+v"(x[3].v));
+    } else if constexpr (!tr<T>::C && N == 8) {
+        asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x[0].v), "+v"(x[1].v), "+v"(x[2].v), "+v"(x[3].v), "+v"(x[4].v),
+                     "+v"(x[5].v), "+v"(x[6].v), "+v"(x[7].v));
+    } else if constexpr (tr<T>::C && N == 2) {
+        asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x[0].re), "+v"(x[0].im), "+v"(x[1].re), "+v"(x[1].im));
+    } else if constexpr (tr<T>::C && N == 4) {
+        asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x[0].re), "+v"(x[0].im), "+v"(x[1].re), "+v"(x[1].im), "+v"(x[2].re),
+                     "+v"(x[2].im), "+v"(x[3].re), "+v"(x[3].im));
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) tile_settle_v(x[i]);
     }
 #else
     (void)x;
