@@ -9,7 +9,7 @@
 //   (b = 256 and complex FP64 at b = 128: the same stages with the factor state in global
 //   memory -- k_factor_gm, k_sweep_gm, k_recover_gm, k_red_setup_gm)
 //   per RHS chunk: y tips keeping the forward sweep (k_sweep), block-Jacobi reduced solve in
-//              FP64 (k_red_jacobi_q / k_red_jacobi), recovery as one backward chain into the FP64
+//              FP64 (k_red_jacobi), recovery as one backward chain into the FP64
 //              solution (k_recover), FP64 residual (k_residual); mixed precision repeats on the
 //              residual until every column meets tol.                                -- solve
 // The reference's flow is OpenMP/spike_interfaces.c:43-419; partition rows follow
@@ -618,7 +618,8 @@ struct Engine {
     int factor();
     int reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, int ymax);
     int direct_pass(Group &g, int ymax);
-    int launch_jacobi(Group &g, int ncc, int ymax, const DevBuf &xo, DevBuf &xn);
+    int jacobi_tiles(int nt, int ymax) const;
+    int launch_jacobi(Group &g, int ct, int ymax, bool first, const DevBuf &xo, DevBuf &xn);
     int run_passes(int ymax, bool capture, double rtol, int max_refine, double &t_y, double &t_red, double &t_rec,
                    double &t_res, double &t_norm, int &passes);
     int read_stats(bool *incomplete = nullptr);
@@ -1517,16 +1518,8 @@ int Engine::run_passes(int ymax, bool capture, double rtol, int max_refine, doub
         for (int gi = 0; gi < ngroups; ++gi) {
             Group &g = *groups[gi];
             if (g.ifs.empty()) continue;
-            const int nif = (int)g.ifs.size(), ngs = (int)g.sys.size();
-            const int ncc = ceil_div(ymax, 16);
-            const int slot = 2 * g.b * ymax;
-            const dim3 zg((unsigned)std::min(nif, 65536));
-            if (dtype == SPIKE_DTYPE_Z)
-                hipLaunchKernelGGL(k_red_zero<zd>, zg, dim3(256), 0, s, (const IfaceDesc *)g.d_ifs.p, nif,
-                                   (const int *)g.d_active.p, g.red0.as<zd>(), slot);
-            else
-                hipLaunchKernelGGL(k_red_zero<double>, zg, dim3(256), 0, s, (const IfaceDesc *)g.d_ifs.p, nif,
-                                   (const int *)g.d_active.p, g.red0.as<double>(), slot);
+            const int ngs = (int)g.sys.size();
+            const int ct = jacobi_tiles(g.NT, ymax), ncc = ceil_div(ymax, 16 * ct);
             hipLaunchKernelGGL(k_red_begin, dim3((ngs + 255) / 256), dim3(256), 0, s, g.d_sysstat.as<SysStat>(), ngs,
                                (const SysDev *)g.d_sysdev.p, (const int *)g.d_active.p, (const int *)g.d_direct.p,
                                g.d_red_active.as<int>());
@@ -1539,7 +1532,7 @@ int Engine::run_passes(int ymax, bool capture, double rtol, int max_refine, doub
                 for (int rep = 0; rep < 2; ++rep) {
                     const DevBuf &xo = rep == 0 ? g.red0 : g.red1;
                     DevBuf &xn = rep == 0 ? g.red1 : g.red0;
-                    if ((e = launch_jacobi(g, ncc, ymax, xo, xn))) return e;
+                    if ((e = launch_jacobi(g, ct, ymax, pr == 0 && rep == 0, xo, xn))) return e;
                 }
                 hipLaunchKernelGGL(k_red_check, dim3((unsigned)ngs), dim3(64), 0, s, g.d_sysstat.as<SysStat>(), ngs,
                                    (const SysDev *)g.d_sysdev.p, (const int *)g.d_part_iface.p, (const double *)g.conv.p,
@@ -1647,44 +1640,27 @@ int Engine::direct_pass(Group &g, int ymax) {
     return reduced_direct(g, which, g.red0, ymax);
 }
 
-int Engine::launch_jacobi(Group &g, int ncc, int ymax, const DevBuf &xo, DevBuf &xn) {
-    hipStream_t s = stream;
+// column tiles per sweep workgroup: enough for the chunk's columns, within the LDS (jacobi_ct)
+int Engine::jacobi_tiles(int nt, int ymax) const {
+    const int need = ymax <= 16 ? 1 : (ymax <= 32 ? 2 : 4);
+    return std::min(need, jacobi_ct((int)h_bytes(dtype), nt));
+}
+
+int Engine::launch_jacobi(Group &g, int ct, int ymax, bool first, const DevBuf &xo, DevBuf &xn) {
+    const int ncc = ceil_div(ymax, 16 * ct);
     const unsigned nb = (unsigned)(g.ifs.size() * ncc);
-    if (g.NT == 16) {               // column sub-chunks keep three b x CK vectors within the LDS
-        if (dtype == SPIKE_DTYPE_Z)
-            hipLaunchKernelGGL((k_red_jacobi<zd, 16, 8>), dim3(nb), dim3(256), 0, s, g.d_ifs.as<IfaceDesc>(), ncc,
-                               (const zd *)g.vt.p, (const zd *)g.vb.p, (const zd *)g.wt.p, (const zd *)g.wb.p,
-                               (const zd *)g.yt.p, (const zd *)g.yb.p, (const zd *)g.T.p, (const zd *)xo.p, xn.as<zd>(),
-                               g.conv.as<double>(), ymax, ymax, g.d_red_active.as<int>());
-        else
-            hipLaunchKernelGGL((k_red_jacobi<double, 16, 16>), dim3(nb), dim3(256), 0, s, g.d_ifs.as<IfaceDesc>(), ncc,
-                               (const double *)g.vt.p, (const double *)g.vb.p, (const double *)g.wt.p,
-                               (const double *)g.wb.p, (const double *)g.yt.p, (const double *)g.yb.p,
-                               (const double *)g.T.p, (const double *)xo.p, xn.as<double>(), g.conv.as<double>(), ymax,
-                               ymax, g.d_red_active.as<int>());
-    } else if (dtype == SPIKE_DTYPE_Z) {
-        NT_SWITCH(g.NT, {
-            hipLaunchKernelGGL((k_red_jacobi<zd, NT, 16>), dim3(nb), dim3(256), 0, s, g.d_ifs.as<IfaceDesc>(), ncc, (const zd *)g.vt.p,
-                               (const zd *)g.vb.p, (const zd *)g.wt.p, (const zd *)g.wb.p, (const zd *)g.yt.p, (const zd *)g.yb.p,
-                               (const zd *)g.T.p, (const zd *)xo.p, xn.as<zd>(), g.conv.as<double>(), ymax, ymax,
-                               g.d_red_active.as<int>());
-        });
-    } else {
-        NT_SWITCH(g.NT, {
-            if constexpr (NT <= 4)
-                hipLaunchKernelGGL((k_red_jacobi_q<double, NT>), dim3(nb), dim3(NT * 64), 0, s, g.d_ifs.as<IfaceDesc>(), ncc,
-                                   (const double *)g.vt.p, (const double *)g.vb.p, (const double *)g.wt.p,
-                                   (const double *)g.wb.p, (const double *)g.yt.p, (const double *)g.yb.p,
-                                   (const double *)g.T.p, (const double *)xo.p, xn.as<double>(), g.conv.as<double>(), ymax,
-                                   ymax, g.d_red_active.as<int>());
-            else
-                hipLaunchKernelGGL((k_red_jacobi<double, NT, 16>), dim3(nb), dim3(256), 0, s, g.d_ifs.as<IfaceDesc>(), ncc,
-                                   (const double *)g.vt.p, (const double *)g.vb.p, (const double *)g.wt.p,
-                                   (const double *)g.wb.p, (const double *)g.yt.p, (const double *)g.yb.p,
-                                   (const double *)g.T.p, (const double *)xo.p, xn.as<double>(), g.conv.as<double>(), ymax,
-                                   ymax, g.d_red_active.as<int>());
-        });
-    }
+    auto launch = [&](auto hz, auto ntc, auto ctc) {
+        typedef decltype(hz) H;
+        constexpr int NT = decltype(ntc)::value, CT = decltype(ctc)::value;
+        if constexpr (CT <= jacobi_ct((int)sizeof(H), NT))
+            hipLaunchKernelGGL((k_red_jacobi<H, NT, CT>), dim3(nb), dim3(NT * 64), 0, stream, (const IfaceDesc *)g.d_ifs.p, ncc,
+                               (const H *)g.vt.p, (const H *)g.vb.p, (const H *)g.wt.p, (const H *)g.wb.p,
+                               (const H *)g.yt.p, (const H *)g.yb.p, (const H *)g.T.p, (const H *)xo.p, xn.as<H>(),
+                               g.conv.as<double>(), ymax, first ? 1 : 0, (const int *)g.d_red_active.p);
+    };
+#define JACOBI_LAUNCH(H) NTA_SWITCH(g.NT, CT_SWITCH(ct, { launch(H(), std::integral_constant<int, NT>(), std::integral_constant<int, CT>()); }))
+    if (dtype == SPIKE_DTYPE_Z) JACOBI_LAUNCH(zd) else JACOBI_LAUNCH(double);
+#undef JACOBI_LAUNCH
     HIPCK(hipGetLastError());
     return SPIKE_SUCCESS;
 }
