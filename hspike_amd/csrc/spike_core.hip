@@ -411,7 +411,11 @@ extern "C" int spike_autotune_partitions_tuned(int n, int ku, int kl, int nrhs, 
         const long x = v ? atol(v) : 0;
         return x > 0 ? x : 96L;
     }();
-    const long blocks_per_part = tune == SPIKE_TUNE_THROUGHPUT ? bpp_throughput : bpp_latency;
+    long blocks_per_part = tune == SPIKE_TUNE_THROUGHPUT ? bpp_throughput : bpp_latency;
+    // the wide groups take a whole CU per partition and about 0.3 ms per 256-row block: three blocks per
+    // partition (n = 60001, k = 200, 16 columns, ms per step: 12 blocks 9.4, 4 blocks 5.29, 3 blocks
+    // 4.80; 2 blocks 3.94, but the couplings of weakly dominant matrices would then need many sweeps)
+    if (wide_group(type_code(dtype, precision), NT)) blocks_per_part = std::min(blocks_per_part, 3L);
     const long rows_target = blocks_per_part * b;
     long P = n / rows_target;
     const long slots = factor_slots(type_code(dtype, precision), NT);

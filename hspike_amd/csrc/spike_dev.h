@@ -263,6 +263,10 @@ template <typename T, int N> __device__ __forceinline__ void tiles_settle_v(Tile
     } else if constexpr (!tr<T>::C && N == 8) {
         asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x[0].v), "+v"(x[1].v), "+v"(x[2].v), "+v"(x[3].v), "+v"(x[4].v),
                      "+v"(x[5].v), "+v"(x[6].v), "+v"(x[7].v));
+    } else if constexpr (!tr<T>::C && N == 16) {
+        asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x[0].v), "+v"(x[1].v), "+v"(x[2].v), "+v"(x[3].v), "+v"(x[4].v),
+                     "+v"(x[5].v), "+v"(x[6].v), "+v"(x[7].v), "+v"(x[8].v), "+v"(x[9].v), "+v"(x[10].v), "+v"(x[11].v),
+                     "+v"(x[12].v), "+v"(x[13].v), "+v"(x[14].v), "+v"(x[15].v));
     } else if constexpr (tr<T>::C && N == 2) {
         asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x[0].re), "+v"(x[0].im), "+v"(x[1].re), "+v"(x[1].im));
     } else if constexpr (tr<T>::C && N == 4) {
