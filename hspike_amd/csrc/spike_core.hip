@@ -1108,6 +1108,52 @@ int Engine::factor() {
 }
 
 // ============================================================================ direct reduced solve
+// Band LU of nd systems whose lower bandwidth is at most klmax: blocked where its LDS holds the
+// multipliers, else column by column (lds: that kernel's dynamic LDS).
+template <typename H>
+int launch_gbtrf(int nd, int klmax, size_t lds, hipStream_t s, const BandSys *sys, H *ab, int *piv, int *info) {
+    if (klmax <= GB_KL_MAX) {
+        const size_t need = gb_blk_lds<H>(klmax);
+        HIPCK(hipFuncSetAttribute((const void *)k_gbtrf_blk<H>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gb_blk_lds<H>(GB_KL_MAX)));
+        hipLaunchKernelGGL(k_gbtrf_blk<H>, dim3(nd), dim3(GB_BTHREADS), need, s, sys, ab, piv, info);
+    } else {
+        hipLaunchKernelGGL(k_gbtrf<H>, dim3(nd), dim3(GB_THREADS), lds, s, sys, ab, piv, info);
+    }
+    HIPCK(hipGetLastError());
+    return SPIKE_SUCCESS;
+}
+
+// Register slots (64 rows each) a wave needs for bandwidth k, rounded up to a built size; 0 where the
+// window does not fit the registers (k_gbtrs takes those)
+template <typename H> int trs_slots(int k) {
+    const int need = 1 + ceil_div(k, 64);
+    for (int s : {2, 4, 8, 16})
+        if (s >= need && s * (int)sizeof(H) <= 128) return s;
+    return 0;
+}
+
+// forward and backward band solves, one wave per item (system, column, 1)
+template <typename H>
+int launch_trs_waves(int nitems, int sf, int sb, hipStream_t s, const BandSys *sys, const int *items, const H *ab,
+                     const int *piv, H *x) {
+    auto go = [&](auto sc, bool fwd) {
+        constexpr int S = decltype(sc)::value;
+        if constexpr (S * (int)sizeof(H) <= 128) {
+            if (fwd) hipLaunchKernelGGL((k_gbtrs_fwd<H, S>), dim3(nitems), dim3(64), 0, s, sys, items, ab, piv, x);
+            else hipLaunchKernelGGL((k_gbtrs_bwd<H, S>), dim3(nitems), dim3(64), 0, s, sys, items, ab, x);
+        }
+    };
+    for (int dir = 0; dir < 2; ++dir)
+        switch (dir == 0 ? sf : sb) {
+        case 2: go(std::integral_constant<int, 2>(), dir == 0); break;
+        case 4: go(std::integral_constant<int, 4>(), dir == 0); break;
+        case 8: go(std::integral_constant<int, 8>(), dir == 0); break;
+        default: go(std::integral_constant<int, 16>(), dir == 0); break;
+        }
+    HIPCK(hipGetLastError());
+    return SPIKE_SUCCESS;
+}
+
 // R of the group-local systems `which` (assembled and factored once per factorization; the set
 // only grows between factorizations), its right-hand side from the RHS tips of this pass, the
 // band solve, and the solution scattered into the interface iterate `xo` the recovery reads.
@@ -1123,7 +1169,7 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
         g.rd_bs.assign(nd, BandSys{});
         g.rd_desc_h.assign(nd, RedDirect{});
         int64_t ab = 0, pv = 0;
-        int maxP = 1;
+        int maxP = 1, klmax = 0;
         size_t lds = 0;
         for (int q = 0; q < nd; ++q) {
             const SysHost &S = sys[g.sys[g.rd_sys[q]]];
@@ -1140,6 +1186,7 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
             D.iface0 = g.part_iface[D.part0];
             D.P = S.P; D.ku = S.ku; D.kl = S.kl; D.band = q;
             maxP = std::max(maxP, S.P);
+            klmax = std::max(klmax, klr);
             lds = std::max(lds, (size_t)(std::max(klr, 1) + klr + kur + 1) * hs);
         }
         if (lds > 64 * 1024) {
@@ -1158,14 +1205,16 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
             hipLaunchKernelGGL(k_red_band<zd>, dim3(maxP, nd), dim3(256), 0, s, g.rd_desc.as<RedDirect>(), g.rd_bsd.as<BandSys>(),
                                (const zd *)g.vt.p, (const zd *)g.vb.p, (const zd *)g.wt.p, (const zd *)g.wb.p, g.b,
                                g.rd_ab.as<zd>());
-            hipLaunchKernelGGL(k_gbtrf<zd>, dim3(nd), dim3(GB_THREADS), lds, s, g.rd_bsd.as<BandSys>(), g.rd_ab.as<zd>(),
-                               g.rd_piv.as<int>(), g.rd_info.as<int>());
+            if ((e = launch_gbtrf<zd>(nd, klmax, lds, s, g.rd_bsd.as<BandSys>(), g.rd_ab.as<zd>(), g.rd_piv.as<int>(),
+                                      g.rd_info.as<int>())))
+                return e;
         } else {
             hipLaunchKernelGGL(k_red_band<double>, dim3(maxP, nd), dim3(256), 0, s, g.rd_desc.as<RedDirect>(),
                                g.rd_bsd.as<BandSys>(), (const double *)g.vt.p, (const double *)g.vb.p,
                                (const double *)g.wt.p, (const double *)g.wb.p, g.b, g.rd_ab.as<double>());
-            hipLaunchKernelGGL(k_gbtrf<double>, dim3(nd), dim3(GB_THREADS), lds, s, g.rd_bsd.as<BandSys>(),
-                               g.rd_ab.as<double>(), g.rd_piv.as<int>(), g.rd_info.as<int>());
+            if ((e = launch_gbtrf<double>(nd, klmax, lds, s, g.rd_bsd.as<BandSys>(), g.rd_ab.as<double>(),
+                                          g.rd_piv.as<int>(), g.rd_info.as<int>())))
+                return e;
         }
         HIPCK(hipGetLastError());
         std::vector<int> info(nd);
@@ -1185,6 +1234,11 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
     std::vector<RedDirect> pass;
     const size_t lds_cap = 48 * 1024;
     size_t lds = 0;
+    int klm = 0, kvm = 0;
+    for (const BandSys &B : g.rd_bs) { klm = std::max(klm, B.kl); kvm = std::max(kvm, B.kl + B.ku); }
+    const int sf = dtype == SPIKE_DTYPE_Z ? trs_slots<zd>(klm) : trs_slots<double>(klm);
+    const int sb = dtype == SPIKE_DTYPE_Z ? trs_slots<zd>(kvm) : trs_slots<double>(kvm);
+    const bool waves = sf && sb;
     for (int q = 0; q < nd; ++q) {
         if (std::find(which.begin(), which.end(), g.rd_sys[q]) == which.end()) continue;
         pass.push_back(g.rd_desc_h[q]);
@@ -1194,7 +1248,9 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
         maxnr = std::max(maxnr, B.n);
         nrow = std::max(nrow, (g.rd_desc_h[q].P - 1) * (g.rd_desc_h[q].ku + g.rd_desc_h[q].kl) * ymax);
         const size_t per_col = (size_t)B.n * hs;
-        if (per_col <= lds_cap) {
+        if (waves) {
+            for (int c = 0; c < ymax; ++c) items.insert(items.end(), {q, c, 1});
+        } else if (per_col <= lds_cap) {
             const int mc = (int)std::min<size_t>({64, (size_t)ymax, lds_cap / per_col});
             for (int c = 0; c < ymax; c += mc) items.insert(items.end(), {q, c, std::min(mc, ymax - c)});
             lds = std::max(lds, per_col * mc);
@@ -1217,7 +1273,11 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
     if (dtype == SPIKE_DTYPE_Z) {
         hipLaunchKernelGGL(k_red_rhs<zd>, dim3(rgrid, npass), dim3(256), 0, s, g.rd_pass.as<RedDirect>(), g.rd_bsd.as<BandSys>(),
                            (const zd *)g.yt.p, (const zd *)g.yb.p, g.b, ymax, g.rd_x.as<zd>());
-        if (ni) hipLaunchKernelGGL((k_gbtrs<zd, true>), dim3(ni), dim3(256), lds, s, g.rd_bsd.as<BandSys>(), g.rd_items.as<int>(),
+        if (waves) {
+            if ((e = launch_trs_waves<zd>(ni, sf, sb, s, g.rd_bsd.as<BandSys>(), g.rd_items.as<int>(), (const zd *)g.rd_ab.p,
+                                          (const int *)g.rd_piv.p, g.rd_x.as<zd>())))
+                return e;
+        } else if (ni) hipLaunchKernelGGL((k_gbtrs<zd, true>), dim3(ni), dim3(256), lds, s, g.rd_bsd.as<BandSys>(), g.rd_items.as<int>(),
                                    (const zd *)g.rd_ab.p, (const int *)g.rd_piv.p, g.rd_x.as<zd>());
         if (ng) hipLaunchKernelGGL((k_gbtrs<zd, false>), dim3(ng), dim3(256), 0, s, g.rd_bsd.as<BandSys>(),
                                    g.rd_items.as<int>() + 3 * ni, (const zd *)g.rd_ab.p, (const int *)g.rd_piv.p,
@@ -1228,7 +1288,11 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
         hipLaunchKernelGGL(k_red_rhs<double>, dim3(rgrid, npass), dim3(256), 0, s, g.rd_pass.as<RedDirect>(),
                            g.rd_bsd.as<BandSys>(), (const double *)g.yt.p, (const double *)g.yb.p, g.b, ymax,
                            g.rd_x.as<double>());
-        if (ni) hipLaunchKernelGGL((k_gbtrs<double, true>), dim3(ni), dim3(256), lds, s, g.rd_bsd.as<BandSys>(),
+        if (waves) {
+            if ((e = launch_trs_waves<double>(ni, sf, sb, s, g.rd_bsd.as<BandSys>(), g.rd_items.as<int>(),
+                                              (const double *)g.rd_ab.p, (const int *)g.rd_piv.p, g.rd_x.as<double>())))
+                return e;
+        } else if (ni) hipLaunchKernelGGL((k_gbtrs<double, true>), dim3(ni), dim3(256), lds, s, g.rd_bsd.as<BandSys>(),
                                    g.rd_items.as<int>(), (const double *)g.rd_ab.p, (const int *)g.rd_piv.p,
                                    g.rd_x.as<double>());
         if (ng) hipLaunchKernelGGL((k_gbtrs<double, false>), dim3(ng), dim3(256), 0, s, g.rd_bsd.as<BandSys>(),
@@ -2271,13 +2335,22 @@ int band_residual(int dtype, int n, const int *rowptr, const int *colind, const 
 int band_trs(int dtype, int n, int ku, int kl, int nrhs, void *p, int ldp, const BandWork &w, hipStream_t st) {
     const size_t hs = h_bytes(dtype), per_col = (size_t)n * hs, cap = 48 * 1024;
     const bool lx = per_col <= cap;
-    const int mc = lx ? (int)std::min<size_t>({64, (size_t)nrhs, cap / per_col}) : std::min(64, nrhs);
+    const int sf = dtype == SPIKE_DTYPE_Z ? trs_slots<zd>(kl) : trs_slots<double>(kl);
+    const int sb = dtype == SPIKE_DTYPE_Z ? trs_slots<zd>(kl + ku) : trs_slots<double>(kl + ku);
+    const bool waves = sf && sb;
+    const int mc = waves ? 1 : (lx ? (int)std::min<size_t>({64, (size_t)nrhs, cap / per_col}) : std::min(64, nrhs));
     BandSys B{};
     B.n = n; B.kl = kl; B.ku = ku; B.ldab = 2 * kl + ku + 1; B.m = nrhs; B.ldx = ldp; B.ab = 0; B.piv = 0; B.x = 0;
     const int ni = (nrhs + mc - 1) / mc;
     hipLaunchKernelGGL(k_put<BandSys>, dim3(1), dim3(64), 0, st, w.sys, B);
     hipLaunchKernelGGL(k_band_items, dim3((ni + 255) / 256), dim3(256), 0, st, w.items, nrhs, mc);
     const size_t lds = lx ? per_col * mc : 0;
+    if (waves && dtype == SPIKE_DTYPE_Z)
+        return launch_trs_waves<zd>(ni, sf, sb, st, (const BandSys *)w.sys, (const int *)w.items, (const zd *)w.ab,
+                                    (const int *)w.piv, (zd *)p);
+    if (waves)
+        return launch_trs_waves<double>(ni, sf, sb, st, (const BandSys *)w.sys, (const int *)w.items, (const double *)w.ab,
+                                        (const int *)w.piv, (double *)p);
     if (dtype == SPIKE_DTYPE_Z) {
         if (lx) hipLaunchKernelGGL((k_gbtrs<zd, true>), dim3(ni), dim3(256), lds, st, (const BandSys *)w.sys, (const int *)w.items,
                                    (const zd *)w.ab, (const int *)w.piv, (zd *)p);
@@ -2318,14 +2391,12 @@ int band_run(int dtype, int n, int ku, int kl, const int *rowptr, const int *col
         hipLaunchKernelGGL(k_fill<zd>, dim3(fg), dim3(256), 0, st, (zd *)w.ab, (int64_t)elems, s_zero_host<zd>());
         hipLaunchKernelGGL(k_csr_to_band<zd>, dim3(rg), dim3(256), 0, st, rowptr, colind, (const zd *)aij, n, kl, ku, ldab,
                            (zd *)w.ab);
-        hipLaunchKernelGGL(k_gbtrf<zd>, dim3(1), dim3(GB_THREADS), lds_f, st, (const BandSys *)w.sys, (zd *)w.ab, w.piv,
-                           w.flags + 3);
+        if (int e = launch_gbtrf<zd>(1, kl, lds_f, st, (const BandSys *)w.sys, (zd *)w.ab, w.piv, w.flags + 3)) return e;
     } else {
         hipLaunchKernelGGL(k_fill<double>, dim3(fg), dim3(256), 0, st, (double *)w.ab, (int64_t)elems, 0.0);
         hipLaunchKernelGGL(k_csr_to_band<double>, dim3(rg), dim3(256), 0, st, rowptr, colind, (const double *)aij, n, kl, ku,
                            ldab, (double *)w.ab);
-        hipLaunchKernelGGL(k_gbtrf<double>, dim3(1), dim3(GB_THREADS), lds_f, st, (const BandSys *)w.sys, (double *)w.ab,
-                           w.piv, w.flags + 3);
+        if (int e = launch_gbtrf<double>(1, kl, lds_f, st, (const BandSys *)w.sys, (double *)w.ab, w.piv, w.flags + 3)) return e;
     }
     HIPCK(hipGetLastError());
     int info = 0;

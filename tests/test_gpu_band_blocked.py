@@ -1,0 +1,64 @@
+"""The blocked band LU and the register-window band solves (k_gbtrf_blk, k_gbtrs_fwd / _bwd) through
+spike_band_solve_host: orders around the panel width (32, complex 16) and the 64-row windows, one-sided
+and empty bands, bandwidths at the edges of the register windows, interchanges over the whole lower
+band, and a band too wide for the blocked kernels (kl > 448), which the column kernels take.
+
+The matrices have singular values >= 1.2 and norms <= 2.8 (a permutation of 2 I inside the band plus
+noise with row sums <= 0.8), so after the FP64 refinement the residual is at rounding level: 1e-14,
+and the solution agrees with the oracle's band LU within 1e-12."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hs():
+    import hspike_amd
+    hspike_amd.load()
+    return hspike_amd
+
+
+def pivoting_band(hs, n, ku, kl, seed, cplx):
+    """2 at (i, s(i)), s reversing groups of min(ku, kl) + 1 rows; zero diagonal where s(i) != i."""
+    rng = np.random.default_rng(seed)
+    i = np.repeat(np.arange(n), ku + kl + 1)
+    j = i + np.tile(np.arange(-kl, ku + 1), n)
+    keep = (j >= 0) & (j < n)
+    i, j = i[keep], j[keep]
+    v = rng.uniform(-1, 1, i.size) * (0.8 / max(ku + kl, 1))
+    if cplx:
+        v = v * np.exp(2j * np.pi * rng.uniform(0, 1, i.size))
+    m = min(ku, kl) + 1
+    first = (i // m) * m
+    to = np.where(first + m <= n, 2 * first + m - 1 - i, i)
+    v[(j == i) & (to != i)] = 0.0
+    v[j == to] = 2.0
+    rp = np.zeros(n + 1, dtype=np.int32)
+    np.add.at(rp, i + 1, 1)
+    return hs.CSRMatrix(n, np.cumsum(rp).astype(np.int32), j.astype(np.int32), v)
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("n,ku,kl,nrhs", [
+    (2, 1, 1, 1), (15, 0, 3, 2), (16, 3, 0, 1), (31, 30, 30, 1), (32, 5, 2, 3), (33, 2, 7, 1), (64, 15, 16, 2), (65, 16, 15, 1),
+    (129, 63, 63, 2), (200, 64, 64, 3), (300, 65, 100, 1), (500, 191, 60, 2), (700, 100, 191, 17), (1000, 250, 192, 1),
+    (1100, 20, 448, 1), (1200, 10, 460, 2),
+])
+def test_band_solve_matches_oracle(hs, oracle_mod, n, ku, kl, nrhs, cplx):
+    A = pivoting_band(hs, n, ku, kl, seed=n + ku, cplx=cplx)
+    B = hs.gen_dense(n, nrhs, seed=3, complex=cplx)
+    X, rel = hs.band_solve(A, B)
+    assert rel.max() <= 1e-14, rel
+    Xo = oracle_mod.direct_solve(oracle_mod.CSR(A.n, A.rowptr, A.colind, A.aij), B)
+    assert np.linalg.norm(X - Xo) / np.linalg.norm(Xo) <= 1e-12
+
+
+@pytest.mark.parametrize("col", [0, 31, 32, 77, 99])
+def test_zero_column_is_singular(hs, col):
+    A = pivoting_band(hs, 100, 4, 6, seed=1, cplx=False)
+    aij = np.where(A.colind == col, 0.0, A.aij)
+    with pytest.raises(hs.SpikeError) as ex:
+        hs.band_solve(hs.CSRMatrix(A.n, A.rowptr, A.colind, aij), np.ones((100, 1)))
+    assert ex.value.code == -4
+    assert "column %d" % col in str(ex.value)
