@@ -476,6 +476,7 @@ struct Group {
     int n_items_vw = 0, n_items_y = 0, n_items_r = 0;
     int ct_vw = 4, ct_y = 1;                // column tiles per sweep workgroup (V/W items, RHS items)
     int ymax = 0;
+    int res_kernels = 1;                    // residual kernels its systems use (launch_residual)
     std::vector<uint64_t> solve_key;        // descriptors of the last solve chunk (reused when equal)
     std::vector<uint64_t> plan_key;         // members, sizes, bandwidths, P and CSR arrays of the plan
     bool plan_uploaded = false;             // d_parts .. d_sysdev hold this plan
@@ -683,12 +684,40 @@ void launch_recover(int nitems, hipStream_t s, const SweepItem *items, const Par
                            part_iface, ymax, (const Q4<T> *)wsave, accumulate, active, wstop);
 }
 
+// The residual kernel of a system, from the system and its columns in the chunk alone (a system gets the
+// same bits alone and in a batch).  The dense-tile kernel costs about the same whatever the fill and
+// reads x once per 16 rows, the gather kernel's time follows the nonzeros and the columns.  us per
+// residual, gather / dense tile (real values):
+//   k = 16, 600000 rows, 15% / 50% fill: 4 columns 49 / 47, 70 / 54; 16 columns 116 / 65, 153 / 87
+//   k = 30, 500000 rows: 4 columns 51 / 67, 101 / 81; 16 columns 109 / 78, 170 / 97
+//   k = 64, 400000 rows: 4 columns 60 / 97, 172 / 144; 16 columns 110 / 102, 224 / 157
+//   k = 100, 300000 rows: 16 columns 108 / 155, 251 / 252; 32 columns 204 / 220, 424 / 317; 64 370 / 350, 771 / 440
+// so: b = 16 always; b = 32 and 64 from 9 columns or a third of the band filled; b = 128 from 33 columns,
+// or from 17 with a quarter filled.
+bool dense_residual(int dtype, int nt, int n, int64_t nnz, int ku, int kl, int m) {
+    if (dtype != SPIKE_DTYPE_D || nt > 8) return false;
+    const double fill = (double)nnz / ((double)n * (ku + kl + 1));
+    if (nt == 1) return true;
+    if (nt <= 4) return m > 8 || fill >= 1.0 / 3;
+    return m > 32 || (m > 16 && fill >= 0.25);
+}
+
 // FP64 residual with TW column lanes per row: the narrowest of 4, 8, 16 covering the chunk's
 // columns (all chunks share the partials stride `ymax`)
 // (TW lanes per row, CPL columns per lane): pairs of columns per lane when the solver keeps the
 // row-major iterate (row stride even), and the fewest lanes per row that cover the columns
-int launch_residual(int dtype, int mcols, int ymax, bool rowmajor, unsigned nchunks, hipStream_t s,
+// which: the kernels of the group's systems (1: k_residual, 2: k_residual_mm, 3: both); nt: block size 16 nt
+int launch_residual(int dtype, int which, int nt, int mcols, int ymax, bool rowmajor, unsigned nchunks, hipStream_t s,
                     const RowChunk *chunks, const SysDev *sys, double *partials, const int *active) {
+    if (which & 2) {
+        NT_SWITCH(nt, {
+            if (mcols <= 16) hipLaunchKernelGGL((k_residual_mm<NT, 1>), dim3(nchunks), dim3(256), 0, s, chunks, sys, partials, ymax, active);
+            else if (mcols <= 32) hipLaunchKernelGGL((k_residual_mm<NT, 2>), dim3(nchunks), dim3(256), 0, s, chunks, sys, partials, ymax, active);
+            else hipLaunchKernelGGL((k_residual_mm<NT, 4>), dim3(nchunks), dim3(256), 0, s, chunks, sys, partials, ymax, active);
+        });
+        HIPCK(hipGetLastError());
+    }
+    if (!(which & 1)) return SPIKE_SUCCESS;
     const int cpl = (rowmajor && dtype == SPIKE_DTYPE_D) ? 2 : 1;     // complex pairs cost too many registers
     const int need = (mcols + cpl - 1) / cpl;
     const int tw = need <= 4 ? 4 : (need <= 8 ? 8 : 16);
@@ -1342,10 +1371,11 @@ int Engine::solve_setup(int c0, int ymax, bool &cached_all) {
         for (size_t gs = 0; gs < ngs; ++gs) {
             const SysHost &S = sys[g.sys[gs]];
             key.insert(key.end(), {(uint64_t)(uintptr_t)S.d_b, (uint64_t)S.ldb, (uint64_t)(uintptr_t)S.d_x,
-                                   (uint64_t)S.ldx, (uint64_t)S.nrhs});
+                                   (uint64_t)S.ldx, (uint64_t)S.nrhs, (uint64_t)S.nnz});
         }
         const bool cached = key == g.solve_key;
         size_t roff = 0, xoff = 0;
+        g.res_kernels = 0;
         for (size_t gs = 0; gs < ngs; ++gs) {
             SysHost &S = sys[g.sys[gs]];
             SysDev &sd = g.sysdev[gs];
@@ -1358,6 +1388,8 @@ int Engine::solve_setup(int c0, int ymax, bool &cached_all) {
             sd.rptr = (char *)g.rwork.p + roff * ymax * hs;
             sd.xrm = (char *)g.xrm.p + xoff * hs;
             sd.ldrm = ldrm;
+            sd.dense = dense_residual(dtype, g.NT, S.n, S.nnz, S.ku, S.kl, m) ? 1 : 0;
+            g.res_kernels |= sd.dense ? 2 : 1;
             roff += S.n;
             xoff += (size_t)S.n * ldrm;
             S.refine_iters = 0;
@@ -1476,7 +1508,7 @@ std::vector<uint64_t> Engine::graph_key(int ymax) const {
     for (int gi = 0; gi < ngroups; ++gi) {
         const Group &g = *groups[gi];
         k.insert(k.end(), {(uint64_t)g.NT, (uint64_t)g.tcode, (uint64_t)g.ct_y, (uint64_t)g.n_items_y, (uint64_t)g.n_items_r,
-                           (uint64_t)g.ifs.size(), (uint64_t)g.chunks.size(), (uint64_t)g.sys.size(), (uint64_t)g.ymax});
+                           (uint64_t)g.ifs.size(), (uint64_t)g.chunks.size(), (uint64_t)g.sys.size(), (uint64_t)g.ymax, (uint64_t)g.res_kernels});
         const DevBuf *bufs[] = {&g.D, &g.U, &g.C, &g.R, &g.Wf, &g.Vf, &g.wstop, &g.rstop, &g.Bt, &g.Ct, &g.vt, &g.vb, &g.wt, &g.wb, &g.T,
                                 &g.yt, &g.yb, &g.red0, &g.red1, &g.scratch, &g.partials, &g.norms, &g.conv, &g.rwork,
                                 &g.xrm, &g.d_active, &g.d_red_active, &g.d_sysstat, &g.d_direct, &g.d_summary,
@@ -1660,7 +1692,7 @@ int Engine::run_passes(int ymax, bool capture, double rtol, int max_refine, doub
         // ---- FP64 residual of every column (residual launches timed apart from the norm sums)
         for (int gi = 0; gi < ngroups; ++gi) {
             Group &g = *groups[gi];
-            if ((e = launch_residual(dtype, ymax, ymax, true, (unsigned)g.chunks.size(), s, g.d_chunks.as<RowChunk>(),
+            if ((e = launch_residual(dtype, g.res_kernels, g.NT, ymax, ymax, true, (unsigned)g.chunks.size(), s, g.d_chunks.as<RowChunk>(),
                                      g.d_sysdev.as<SysDev>(), g.partials.as<double>(), g.d_active.as<int>())))
                 return e;
         }
@@ -2235,7 +2267,7 @@ int residual_dev(int dtype, int n, const int *d_rowptr, const int *d_colind, con
         sd.rptr = (char *)d_r + (size_t)c0 * n * hs;
         int c0s[2] = {0, nch};
         if ((e = upload(ws.dsys, &sd, sizeof sd, st)) || (e = upload(ws.dc0, c0s, sizeof c0s, st))) return e;
-        if ((e = launch_residual(dtype, m, 64, false, (unsigned)nch, st, ws.dch.as<RowChunk>(), ws.dsys.as<SysDev>(),
+        if ((e = launch_residual(dtype, 1, 0, m, 64, false, (unsigned)nch, st, ws.dch.as<RowChunk>(), ws.dsys.as<SysDev>(),
                                  ws.dpart.as<double>(), (const int *)nullptr)))
             return e;
         hipLaunchKernelGGL(k_norm_reduce, dim3(64), dim3(256), 0, st, ws.dc0.as<int>(), ws.dsys.as<SysDev>(),
@@ -2318,7 +2350,7 @@ int band_residual(int dtype, int n, const int *rowptr, const int *colind, const 
         sd.rptr = (char *)r + (size_t)c0 * n * hs;
         hipLaunchKernelGGL(k_put<SysDev>, dim3(1), dim3(64), 0, st, w.sysdev, sd);
         int e;
-        if ((e = launch_residual(dtype, m, 64, false, (unsigned)nch, st, w.chunks, w.sysdev, w.partials, (const int *)nullptr)))
+        if ((e = launch_residual(dtype, 1, 0, m, 64, false, (unsigned)nch, st, w.chunks, w.sysdev, w.partials, (const int *)nullptr)))
             return e;
         hipLaunchKernelGGL(k_norm_reduce, dim3(64), dim3(256), 0, st, (const int *)w.c0s, (const SysDev *)w.sysdev,
                            (const double *)w.partials, w.norms, 64);

@@ -342,7 +342,7 @@ struct SysDev {
     void *rptr;         // residual work (H)
     const void *xrm;    // row-major copy of the solution (row stride ldrm), or null to read xptr
     int ldrm;
-    int pad_;
+    int dense;          // residual kernel of the system: 1 = k_residual_mm, 0 = k_residual
 };
 
 struct RowChunk {
