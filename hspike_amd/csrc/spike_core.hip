@@ -453,6 +453,12 @@ struct SysHost {
 };
 
 struct Group {
+    hipStream_t st = nullptr;               // stream of the group's launches in the current phase (Engine::fork_groups)
+    hipEvent_t sev[6] = {};                 // its factor stages' ends (groups side by side only)
+    ~Group() {
+        for (auto v : sev)
+            if (v) (void)hipEventDestroy(v);
+    }
     int NT = 1, b = 16, tcode = 1;
     std::vector<int> sys;                   // batch indices
     std::vector<PartDesc> parts;
@@ -585,8 +591,57 @@ struct Engine {
         if (events)
             for (auto &e : ev) (void)hipEventDestroy(e);
         if (gexec) (void)hipGraphExecDestroy(gexec);
+        for (auto x : side) { (void)hipStreamSynchronize(x); (void)hipStreamDestroy(x); }
+        for (auto v : side_ev) (void)hipEventDestroy(v);
+        if (fork_ev) (void)hipEventDestroy(fork_ev);
         if (own_stream) (void)hipStreamDestroy(own_stream);
     }
+    // With graph = 1 the block-size groups of a batch run side by side, each on a stream of its own
+    // (their launches are independent, and a group of few or long partitions leaves most of the
+    // device idle): fork_groups orders the groups' streams after the engine's, join_groups the other
+    // way round.  The first group keeps the engine's stream.  With one group, or eager, every group
+    // stays on the engine's stream.
+    std::vector<hipStream_t> side;
+    std::vector<hipEvent_t> side_ev;
+    hipEvent_t fork_ev = nullptr;
+    int init_side() {                       // not under capture: fork_groups then creates nothing
+        if (!fork_ev) HIPCK(hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming));
+        while ((int)side.size() < ngroups - 1) {
+            hipStream_t x = nullptr;
+            HIPCK(hipStreamCreateWithFlags(&x, hipStreamNonBlocking));
+            side.push_back(x);
+        }
+        while (side_ev.size() < side.size()) {
+            hipEvent_t v = nullptr;
+            HIPCK(hipEventCreateWithFlags(&v, hipEventDisableTiming));
+            side_ev.push_back(v);
+        }
+        return 0;
+    }
+    int fork_groups(bool apart) {
+        for (int gi = 0; gi < ngroups; ++gi) groups[gi]->st = stream;
+        if (!apart || ngroups < 2) return 0;
+        HIPCK(hipEventRecord(fork_ev, stream));
+        for (int gi = 1; gi < ngroups; ++gi) {
+            HIPCK(hipStreamWaitEvent(side[gi - 1], fork_ev, 0));
+            groups[gi]->st = side[gi - 1];
+        }
+        return 0;
+    }
+    int join_groups() {
+        for (int gi = 1; gi < ngroups; ++gi)
+            if (groups[gi]->st != stream) {
+                const hipStream_t x = groups[gi]->st;
+                groups[gi]->st = stream;
+                HIPCK(hipEventRecord(side_ev[gi - 1], x));
+                HIPCK(hipStreamWaitEvent(stream, side_ev[gi - 1], 0));
+            }
+        return 0;
+    }
+    struct JoinGuard {                      // an early return leaves no group's launches behind
+        Engine &E;
+        ~JoinGuard() { (void)E.join_groups(); }
+    };
     int init_events() {
         if (events) return 0;
         for (auto &e : ev) HIPCK(hipEventCreate(&e));
@@ -955,6 +1010,22 @@ int Engine::factor() {
         g.plan_uploaded = true;
     }
     HIPCK(hipEventRecord(ev[2], s));
+    const bool apart = o.graph && ngroups > 1;
+    if (apart) {
+        if ((e = init_side())) return e;
+        for (int gi = 0; gi < ngroups; ++gi)
+            for (auto &v : groups[gi]->sev)
+                if (!v) HIPCK(hipEventCreate(&v));
+    }
+    if ((e = fork_groups(apart))) return e;
+    JoinGuard guard{*this};
+    // the end of stage k - 2: one event, or with the groups side by side one of each group's stream
+    auto stage_end = [&](int k) -> int {
+        if (!apart) { HIPCK(hipEventRecord(ev[k], s)); return 0; }
+        for (int gi = 0; gi < ngroups; ++gi) HIPCK(hipEventRecord(groups[gi]->sev[k - 2], groups[gi]->st));
+        return 0;
+    };
+    if (apart && (e = stage_end(2))) return e;
     for (int gi = 0; gi < ngroups; ++gi) {
         Group &g = *groups[gi];
         const int np = (int)g.parts.size();
@@ -963,7 +1034,7 @@ int Engine::factor() {
 #define CONV_LAUNCH                                                                                            \
     {                                                                                                          \
         constexpr int RS = conv_rows((int)sizeof(T), NT);                                                      \
-        hipLaunchKernelGGL((k_csr_to_blocks<T, NT, RS>), dim3((unsigned)((g.nblk * 16 * NT + RS - 1) / RS)), dim3(256), 0, s, \
+        hipLaunchKernelGGL((k_csr_to_blocks<T, NT, RS>), dim3((unsigned)((g.nblk * 16 * NT + RS - 1) / RS)), dim3(256), 0, g.st, \
                            g.blkmap.as<int>(), g.d_sysdev.as<SysDev>(), g.d_parts.as<PartDesc>(), (int64_t)g.nblk, g.D.as<T>(), \
                            wide ? g.Wf.as<T>() : g.U.as<T>(), g.C.as<T>(), g.Bt.as<T>(), g.Ct.as<T>(),         \
                            g.status.as<int>());                                                                \
@@ -974,13 +1045,13 @@ int Engine::factor() {
         HIPCK(hipGetLastError());
         (void)np;
     }
-    HIPCK(hipEventRecord(ev[3], s));
+    if ((e = stage_end(3))) return e;
     for (int gi = 0; gi < ngroups; ++gi) {
         Group &g = *groups[gi];
         const int np = (int)g.parts.size();
         if (wide_group(g.tcode, g.NT)) {
             WIDE_SWITCH(g.tcode, g.NT, {
-                hipLaunchKernelGGL((k_factor_gm<T, NT>), dim3(np), dim3(NT * 64), 0, s, g.d_parts.as<PartDesc>(),
+                hipLaunchKernelGGL((k_factor_gm<T, NT>), dim3(np), dim3(NT * 64), 0, g.st, g.d_parts.as<PartDesc>(),
                                    g.D.as<T>(), g.U.as<T>(), (const T *)g.C.as<T>(), g.R.as<T>(), (const T *)g.Wf.as<T>(),
                                    g.pivinfo.as<double>(), g.rstop.as<int>());
             });
@@ -991,39 +1062,39 @@ int Engine::factor() {
                 bool one = false;
                 if constexpr (factor_one_copy<T, NT>()) one = np > factor_slots(g.tcode, NT);
                 if (one)
-                    hipLaunchKernelGGL((k_factor<T, NT, factor_one_copy<T, NT>() ? 1 : 2>), dim3(np), dim3(NT * 64), 0, s,
+                    hipLaunchKernelGGL((k_factor<T, NT, factor_one_copy<T, NT>() ? 1 : 2>), dim3(np), dim3(NT * 64), 0, g.st,
                                        g.d_parts.as<PartDesc>(), g.D.as<T>(), g.U.as<T>(), (const T *)g.C.as<T>(),
                                        g.R.as<T>(), g.pivinfo.as<double>(), (const int *)nullptr, g.rstop.as<int>());
                 else
-                    hipLaunchKernelGGL((k_factor<T, NT, 2>), dim3(np), dim3(NT * 64), 0, s, g.d_parts.as<PartDesc>(),
+                    hipLaunchKernelGGL((k_factor<T, NT, 2>), dim3(np), dim3(NT * 64), 0, g.st, g.d_parts.as<PartDesc>(),
                                        g.D.as<T>(), g.U.as<T>(), (const T *)g.C.as<T>(), g.R.as<T>(),
                                        g.pivinfo.as<double>(), (const int *)nullptr, g.rstop.as<int>());
             }));
         }
         HIPCK(hipGetLastError());
     }
-    HIPCK(hipEventRecord(ev[4], s));
+    if ((e = stage_end(4))) return e;
     for (int gi = 0; gi < ngroups; ++gi) {
         Group &g = *groups[gi];
         const int np = (int)g.parts.size();
         if (wide_group(g.tcode, g.NT)) continue;          // k_factor_gm forms R
         T_SWITCH(g.tcode, NT_SWITCH(g.NT, {
             if constexpr (!factor_forms_r<T, NT>())        // else the factor kernel formed R
-                hipLaunchKernelGGL((k_rtop<T, NT>), dim3(np), dim3(NT * 64), 0, s, g.d_parts.as<PartDesc>(),
+                hipLaunchKernelGGL((k_rtop<T, NT>), dim3(np), dim3(NT * 64), 0, g.st, g.d_parts.as<PartDesc>(),
                                    (const T *)g.U.as<T>(), g.R.as<T>(), (const int *)nullptr, g.rstop.as<int>());
         }));
         HIPCK(hipGetLastError());
     }
-    HIPCK(hipEventRecord(ev[5], s));
+    if ((e = stage_end(5))) return e;
     // ---- V / W spike tips (partitions of systems with P > 1); wstop starts at zero (fill kernel)
     for (int gi = 0; gi < ngroups; ++gi) {
         Group &g = *groups[gi];
-        if ((e = fill_zero<int>(g.wstop, g.parts.size(), s))) return e;
+        if ((e = fill_zero<int>(g.wstop, g.parts.size(), g.st))) return e;
         if (g.vw_uploaded) {
             if (g.n_items_vw) {
                 T_SWITCH(g.tcode, NTA_SWITCH(g.NT, CT_SWITCH(g.ct_vw, {
                     typedef typename tr<T>::H H;
-                    (launch_sweep<T, NT, CT, true>)(g.n_items_vw, s, g.items_vw.as<SweepItem>(), g.d_parts.as<PartDesc>(),
+                    (launch_sweep<T, NT, CT, true>)(g.n_items_vw, g.st, g.items_vw.as<SweepItem>(), g.d_parts.as<PartDesc>(),
                                             g.D.as<T>(), g.C.as<T>(), g.U.as<T>(), g.R.as<T>(), g.Bt.as<T>(),
                                             g.Ct.as<T>(), g.vt.as<H>(), g.vb.as<H>(), g.wt.as<H>(), g.wb.as<H>(),
                                             (H *)nullptr, (H *)nullptr, g.Wf.as<T>(), g.Vf.as<T>(), (T *)nullptr, 0,
@@ -1051,10 +1122,10 @@ int Engine::factor() {
         g.n_items_vw = (int)items.size();
         g.vw_uploaded = true;
         if (items.empty()) continue;
-        if ((e = upload(g.items_vw, items.data(), items.size() * sizeof(SweepItem), s))) return e;
+        if ((e = upload(g.items_vw, items.data(), items.size() * sizeof(SweepItem), g.st))) return e;
         T_SWITCH(g.tcode, NTA_SWITCH(g.NT, CT_SWITCH(g.ct_vw, {
             typedef typename tr<T>::H H;
-            (launch_sweep<T, NT, CT, true>)(g.n_items_vw, s, g.items_vw.as<SweepItem>(), g.d_parts.as<PartDesc>(),
+            (launch_sweep<T, NT, CT, true>)(g.n_items_vw, g.st, g.items_vw.as<SweepItem>(), g.d_parts.as<PartDesc>(),
                                     g.D.as<T>(), g.C.as<T>(), g.U.as<T>(), g.R.as<T>(), g.Bt.as<T>(),
                                     g.Ct.as<T>(), g.vt.as<H>(), g.vb.as<H>(), g.wt.as<H>(), g.wb.as<H>(),
                                     (H *)nullptr, (H *)nullptr, g.Wf.as<T>(), g.Vf.as<T>(), (T *)nullptr, 0,
@@ -1062,35 +1133,37 @@ int Engine::factor() {
         })));
         HIPCK(hipGetLastError());
     }
-    HIPCK(hipEventRecord(ev[6], s));
+    if ((e = stage_end(6))) return e;
     // ---- reduced-system setup: T_i = (I - Wt_{i+1} Vb_i)^{-1}
     for (int gi = 0; gi < ngroups; ++gi) {
         Group &g = *groups[gi];
         if (g.ifs.empty()) continue;
         if (g.NT == 16) {                                   // global-memory inversion (16-wide panels)
             if (dtype == SPIKE_DTYPE_Z)
-                hipLaunchKernelGGL((k_red_setup_gm<zd, 16>), dim3((unsigned)g.ifs.size()), dim3(16 * 64), 0, s,
+                hipLaunchKernelGGL((k_red_setup_gm<zd, 16>), dim3((unsigned)g.ifs.size()), dim3(16 * 64), 0, g.st,
                                    g.d_ifs.as<IfaceDesc>(), (const zd *)g.vb.p, (const zd *)g.wt.p, g.T.as<zd>(),
                                    g.status.as<int>() + 1, (const int *)nullptr);
             else
-                hipLaunchKernelGGL((k_red_setup_gm<double, 16>), dim3((unsigned)g.ifs.size()), dim3(16 * 64), 0, s,
+                hipLaunchKernelGGL((k_red_setup_gm<double, 16>), dim3((unsigned)g.ifs.size()), dim3(16 * 64), 0, g.st,
                                    g.d_ifs.as<IfaceDesc>(), (const double *)g.vb.p, (const double *)g.wt.p,
                                    g.T.as<double>(), g.status.as<int>() + 1, (const int *)nullptr);
         } else if (dtype == SPIKE_DTYPE_Z) {
             NT_SWITCH(g.NT, {
-                hipLaunchKernelGGL((k_red_setup_mfma<zd, NT>), dim3((unsigned)g.ifs.size()), dim3(NT * 64), 0, s,
+                hipLaunchKernelGGL((k_red_setup_mfma<zd, NT>), dim3((unsigned)g.ifs.size()), dim3(NT * 64), 0, g.st,
                                    g.d_ifs.as<IfaceDesc>(), (const zd *)g.vb.p, (const zd *)g.wt.p, g.T.as<zd>(),
                                    g.status.as<int>() + 1, (const int *)nullptr);
             });
         } else {
             NT_SWITCH(g.NT, {
-                hipLaunchKernelGGL((k_red_setup_mfma<double, NT>), dim3((unsigned)g.ifs.size()), dim3(NT * 64), 0, s,
+                hipLaunchKernelGGL((k_red_setup_mfma<double, NT>), dim3((unsigned)g.ifs.size()), dim3(NT * 64), 0, g.st,
                                    g.d_ifs.as<IfaceDesc>(), (const double *)g.vb.p, (const double *)g.wt.p,
                                    g.T.as<double>(), g.status.as<int>() + 1, (const int *)nullptr);
             });
         }
         HIPCK(hipGetLastError());
     }
+    if (apart && (e = stage_end(7))) return e;
+    if ((e = join_groups())) return e;
     HIPCK(hipEventRecord(ev[7], s));
     // ---- status: malformed entries, singular pivots
     for (int gi = 0; gi < ngroups; ++gi) {
@@ -1127,11 +1200,21 @@ int Engine::factor() {
         if (stv[1]) { set_err("singular reduced-system block%s", ""); return SPIKE_ERR_SINGULAR; }
     }
     factored = true;
-    st.ms_convert = ev_ms(2, 3);
-    st.ms_factor = ev_ms(3, 4);
-    st.ms_rtop = ev_ms(4, 5);
-    st.ms_spikes = ev_ms(5, 6);
-    st.ms_red_setup = ev_ms(6, 7);
+    // a stage of groups side by side: the longest of the groups' times (they overlap)
+    auto stage_ms = [&](int k) -> float {
+        if (!apart) return ev_ms(k - 1, k);
+        float mx = 0.0f;
+        for (int gi = 0; gi < ngroups; ++gi) {
+            float ms = 0.0f;
+            if (hipEventElapsedTime(&ms, groups[gi]->sev[k - 3], groups[gi]->sev[k - 2]) == hipSuccess) mx = std::max(mx, ms);
+        }
+        return mx;
+    };
+    st.ms_convert = stage_ms(3);
+    st.ms_factor = stage_ms(4);
+    st.ms_rtop = stage_ms(5);
+    st.ms_spikes = stage_ms(6);
+    st.ms_red_setup = stage_ms(7);
     st.ms_factor_total = now_ms() - t0;
     return SPIKE_SUCCESS;
 }
@@ -1455,7 +1538,7 @@ int Engine::solve_chunk(int c0, int ymax) {
     double t_y = 0, t_red = 0, t_rec = 0, t_res = 0, t_norm = 0;
     int passes = 0;
     bool cached;
-    if ((e = solve_setup(c0, ymax, cached))) return e;
+    if ((e = solve_setup(c0, ymax, cached)) || (e = fork_groups(false))) return e;
     for (int gi = 0; gi < ngroups; ++gi) {
         Group &g = *groups[gi];
         const int ngs = (int)g.sys.size();
@@ -1540,18 +1623,21 @@ int Engine::solve_graph(int ymax) {
     if (!gexec || key != gkey) {
         if (gexec) { (void)hipGraphExecDestroy(gexec); gexec = nullptr; }
         hipGraph_t graph = nullptr;
+        if (ngroups > 1 && (e = init_side())) return e;
         HIPCK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        int rc = SPIKE_SUCCESS;
+        int rc = fork_groups(true);
         for (int gi = 0; gi < ngroups && !rc; ++gi) {
             Group &g = *groups[gi];
             const int ngs = (int)g.sys.size();
-            hipLaunchKernelGGL(k_stat_init, dim3((ngs + 255) / 256), dim3(256), 0, stream, g.d_sysstat.as<SysStat>(), ngs,
+            hipLaunchKernelGGL(k_stat_init, dim3((ngs + 255) / 256), dim3(256), 0, g.st, g.d_sysstat.as<SysStat>(), ngs,
                                (const SysDev *)g.d_sysdev.p, g.d_active.as<int>(), 1);
             if (hipGetLastError() != hipSuccess) rc = SPIKE_ERR_DEVICE;
         }
         double t_y = 0, t_red = 0, t_rec = 0, t_res = 0, t_norm = 0;
         int passes = 0;
         if (!rc) rc = run_passes(ymax, true, rtol, max_refine, t_y, t_red, t_rec, t_res, t_norm, passes);
+        const int jc = join_groups();
+        if (!rc) rc = jc;
         const hipError_t ce = hipStreamEndCapture(stream, &graph);
         if (rc || ce != hipSuccess) {
             if (graph) (void)hipGraphDestroy(graph);
@@ -1604,7 +1690,7 @@ int Engine::run_passes(int ymax, bool capture, double rtol, int max_refine, doub
             const DevBuf &items = it == 0 ? g.items_yb : g.items_yr;
             T_SWITCH(g.tcode, NTA_SWITCH(g.NT, CT_SWITCH(g.ct_y, {
                 typedef typename tr<T>::H H;
-                (launch_sweep<T, NT, CT, false>)(g.n_items_y, s, items.as<SweepItem>(), g.d_parts.as<PartDesc>(), g.D.as<T>(),
+                (launch_sweep<T, NT, CT, false>)(g.n_items_y, g.st, items.as<SweepItem>(), g.d_parts.as<PartDesc>(), g.D.as<T>(),
                                         g.C.as<T>(), g.U.as<T>(), g.R.as<T>(), g.Bt.as<T>(), g.Ct.as<T>(), (H *)nullptr,
                                         (H *)nullptr, (H *)nullptr, (H *)nullptr, g.yt.as<H>(), g.yb.as<H>(),
                                         (T *)nullptr, (T *)nullptr, g.scratch.as<T>(), g.ymax, g.d_active.as<int>(),
@@ -1620,7 +1706,7 @@ int Engine::run_passes(int ymax, bool capture, double rtol, int max_refine, doub
             if (g.ifs.empty()) continue;
             const int ngs = (int)g.sys.size();
             const int ct = jacobi_tiles(g.NT, ymax), ncc = ceil_div(ymax, 16 * ct);
-            hipLaunchKernelGGL(k_red_begin, dim3((ngs + 255) / 256), dim3(256), 0, s, g.d_sysstat.as<SysStat>(), ngs,
+            hipLaunchKernelGGL(k_red_begin, dim3((ngs + 255) / 256), dim3(256), 0, g.st, g.d_sysstat.as<SysStat>(), ngs,
                                (const SysDev *)g.d_sysdev.p, (const int *)g.d_active.p, (const int *)g.d_direct.p,
                                g.d_red_active.as<int>());
             HIPCK(hipGetLastError());
@@ -1634,7 +1720,7 @@ int Engine::run_passes(int ymax, bool capture, double rtol, int max_refine, doub
                     DevBuf &xn = rep == 0 ? g.red1 : g.red0;
                     if ((e = launch_jacobi(g, ct, ymax, pr == 0 && rep == 0, xo, xn))) return e;
                 }
-                hipLaunchKernelGGL(k_red_check, dim3((unsigned)ngs), dim3(64), 0, s, g.d_sysstat.as<SysStat>(), ngs,
+                hipLaunchKernelGGL(k_red_check, dim3((unsigned)ngs), dim3(64), 0, g.st, g.d_sysstat.as<SysStat>(), ngs,
                                    (const SysDev *)g.d_sysdev.p, (const int *)g.d_part_iface.p, (const double *)g.conv.p,
                                    ncc, rtol, 2 * (pr + 1), g.d_red_active.as<int>());
                 HIPCK(hipGetLastError());
@@ -1681,7 +1767,7 @@ int Engine::run_passes(int ymax, bool capture, double rtol, int max_refine, doub
             const DevBuf &items = it == 0 ? g.items_rb : g.items_rr;
             T_SWITCH(g.tcode, NTA_SWITCH(g.NT, CT_SWITCH(g.ct_y, {
                 typedef typename tr<T>::H H;
-                (launch_recover<T, NT, CT>)(g.n_items_r, s, items.as<SweepItem>(), g.d_parts.as<PartDesc>(), g.U.as<T>(),
+                (launch_recover<T, NT, CT>)(g.n_items_r, g.st, items.as<SweepItem>(), g.d_parts.as<PartDesc>(), g.U.as<T>(),
                                           g.Wf.as<T>(), g.Vf.as<T>(), (const H *)g.red0.p, g.d_part_iface.as<int>(),
                                           g.ymax, g.scratch.as<T>(), it > 0 ? 1 : 0, g.d_active.as<int>(),
                                           (const int *)g.wstop.as<int>());
@@ -1692,7 +1778,7 @@ int Engine::run_passes(int ymax, bool capture, double rtol, int max_refine, doub
         // ---- FP64 residual of every column (residual launches timed apart from the norm sums)
         for (int gi = 0; gi < ngroups; ++gi) {
             Group &g = *groups[gi];
-            if ((e = launch_residual(dtype, g.res_kernels, g.NT, ymax, ymax, true, (unsigned)g.chunks.size(), s, g.d_chunks.as<RowChunk>(),
+            if ((e = launch_residual(dtype, g.res_kernels, g.NT, ymax, ymax, true, (unsigned)g.chunks.size(), g.st, g.d_chunks.as<RowChunk>(),
                                      g.d_sysdev.as<SysDev>(), g.partials.as<double>(), g.d_active.as<int>())))
                 return e;
         }
@@ -1700,9 +1786,9 @@ int Engine::run_passes(int ymax, bool capture, double rtol, int max_refine, doub
         for (int gi = 0; gi < ngroups; ++gi) {
             Group &g = *groups[gi];
             const int ngs = (int)g.sys.size();
-            hipLaunchKernelGGL(k_norm_reduce, dim3((unsigned)(ngs * ymax)), dim3(256), 0, s, g.d_chunk0.as<int>(),
+            hipLaunchKernelGGL(k_norm_reduce, dim3((unsigned)(ngs * ymax)), dim3(256), 0, g.st, g.d_chunk0.as<int>(),
                                g.d_sysdev.as<SysDev>(), g.partials.as<double>(), g.norms.as<double>(), ymax);
-            hipLaunchKernelGGL(k_refine_check, dim3((ngs + 255) / 256), dim3(256), 0, s, g.d_sysstat.as<SysStat>(), ngs,
+            hipLaunchKernelGGL(k_refine_check, dim3((ngs + 255) / 256), dim3(256), 0, g.st, g.d_sysstat.as<SysStat>(), ngs,
                                (const SysDev *)g.d_sysdev.p, (const double *)g.norms.p, ymax, o.tol, it, max_refine,
                                g.d_active.as<int>());
             HIPCK(hipGetLastError());
@@ -1753,7 +1839,7 @@ int Engine::launch_jacobi(Group &g, int ct, int ymax, bool first, const DevBuf &
         typedef decltype(hz) H;
         constexpr int NT = decltype(ntc)::value, CT = decltype(ctc)::value;
         if constexpr (CT <= jacobi_ct((int)sizeof(H), NT))
-            hipLaunchKernelGGL((k_red_jacobi<H, NT, CT>), dim3(nb), dim3(NT * 64), 0, stream, (const IfaceDesc *)g.d_ifs.p, ncc,
+            hipLaunchKernelGGL((k_red_jacobi<H, NT, CT>), dim3(nb), dim3(NT * 64), 0, g.st, (const IfaceDesc *)g.d_ifs.p, ncc,
                                (const H *)g.vt.p, (const H *)g.vb.p, (const H *)g.wt.p, (const H *)g.wb.p,
                                (const H *)g.yt.p, (const H *)g.yb.p, (const H *)g.T.p, (const H *)xo.p, xn.as<H>(),
                                g.conv.as<double>(), ymax, first ? 1 : 0, (const int *)g.d_red_active.p);

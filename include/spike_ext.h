@@ -68,7 +68,10 @@ typedef struct {
  * budget, a system on the direct reduced solve, or any change of the arrays falls back to the
  * eager solve (which sets a new budget).  The handle then works on a non-blocking stream of its
  * own unless spike_set_stream gave one; each call first waits for the default stream.  Per-stage
- * times (ms_ysweep .. ms_norms) are not measured in a replayed solve. */
+ * times (ms_ysweep .. ms_norms) are not measured in a replayed solve.  In a batch of several block
+ * sizes the launches of each block size run on a stream of their own (with graph = 1 only), in the
+ * factorization too: ms_convert .. ms_red_setup are then each the longest of the block sizes' times,
+ * which overlap. */
 
 /* Solver of the reduced system R (stage 3).  AUTO runs block-Jacobi sweeps and switches a
  * system to the direct solver when its sweeps stop contracting (update growing past 1e3 times
