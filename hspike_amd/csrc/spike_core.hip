@@ -1790,8 +1790,13 @@ int Engine::run_passes(int ymax, bool capture, double rtol, int max_refine, doub
         for (int gi = 0; gi < ngroups; ++gi) {
             Group &g = *groups[gi];
             const int ngs = (int)g.sys.size();
+            bool slabs = false;
+            for (int gs = 0; gs < ngs; ++gs) slabs |= g.chunk0[gs + 1] - g.chunk0[gs] > NORM_MIN;
+            if (slabs)
+                hipLaunchKernelGGL(k_norm_slabs, dim3((unsigned)ngs * NORM_SLABS), dim3(256), 0, g.st, g.d_chunk0.as<int>(),
+                                   g.partials.as<double>(), ymax);
             hipLaunchKernelGGL(k_norm_reduce, dim3((unsigned)(ngs * ymax)), dim3(256), 0, g.st, g.d_chunk0.as<int>(),
-                               g.d_sysdev.as<SysDev>(), g.partials.as<double>(), g.norms.as<double>(), ymax);
+                               g.d_sysdev.as<SysDev>(), g.partials.as<double>(), g.norms.as<double>(), ymax, slabs ? 1 : 0);
             hipLaunchKernelGGL(k_refine_check, dim3((ngs + 255) / 256), dim3(256), 0, g.st, g.d_sysstat.as<SysStat>(), ngs,
                                (const SysDev *)g.d_sysdev.p, (const double *)g.norms.p, ymax, o.tol, it, max_refine,
                                g.d_active.as<int>());
@@ -2361,7 +2366,7 @@ int residual_dev(int dtype, int n, const int *d_rowptr, const int *d_colind, con
                                  ws.dpart.as<double>(), (const int *)nullptr)))
             return e;
         hipLaunchKernelGGL(k_norm_reduce, dim3(64), dim3(256), 0, st, ws.dc0.as<int>(), ws.dsys.as<SysDev>(),
-                           ws.dpart.as<double>(), ws.dnorm.as<double>(), 64);
+                           ws.dpart.as<double>(), ws.dnorm.as<double>(), 64, 0);
         HIPCK(hipGetLastError());
         double nr[128];
         HIPCK(hipMemcpyAsync(nr, ws.dnorm.p, sizeof nr, hipMemcpyDeviceToHost, st));
@@ -2443,7 +2448,7 @@ int band_residual(int dtype, int n, const int *rowptr, const int *colind, const 
         if ((e = launch_residual(dtype, 1, 0, m, 64, false, (unsigned)nch, st, w.chunks, w.sysdev, w.partials, (const int *)nullptr)))
             return e;
         hipLaunchKernelGGL(k_norm_reduce, dim3(64), dim3(256), 0, st, (const int *)w.c0s, (const SysDev *)w.sysdev,
-                           (const double *)w.partials, w.norms, 64);
+                           (const double *)w.partials, w.norms, 64, 0);
         HIPCK(hipGetLastError());
         double nr[128];
         HIPCK(hipMemcpyAsync(nr, w.norms, sizeof nr, hipMemcpyDeviceToHost, st));
