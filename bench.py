@@ -248,12 +248,15 @@ def roofline_of(stage_roof, avg_ms):
     return roof
 
 
-def kernel_names_for(nts, nrhs_max, one_copy=()):
+def kernel_names_for(nts, nrhs_max, one_copy=(), fill=1.0):
     """Instantiations the library launches for block sizes 16*NT (FP32 factors) and up to nrhs_max
     RHS columns per chunk (column tiles per sweep workgroup CT with CT * NT <= 16); several block
     sizes are joined with '+'.  `one_copy`: block sizes whose factor launch has more partitions than
-    the device runs at once, so it takes the variant with one LDS copy of R's rows (FP32 b = 64)."""
+    the device runs at once, so it takes the variant with one LDS copy of R's rows (FP32 b = 64).
+    `fill`: filled part of the band, which with the columns decides the residual's kernel."""
     m = min(nrhs_max, 64)
+    dense = lambda nt: nt == 1 or (nt <= 4 and (m > 8 or fill >= 1 / 3)) or (nt == 8 and (m > 32 or (m > 16 and fill >= 0.25)))
+    ncg = 1 if m <= 16 else (2 if m <= 32 else 4)
     ct_max = lambda nt: 4 if 4 * nt * 4 <= 64 else (2 if 2 * nt * 4 <= 64 else 1)   # FP32 sweep tiles
     ct_vw = lambda nt: min(ct_max(nt), nt)           # a spike has at most b = 16 NT columns
     ct_y = lambda nt: min(ct_max(nt), 1 if m <= 16 else (2 if m <= 32 else 4))
@@ -263,7 +266,8 @@ def kernel_names_for(nts, nrhs_max, one_copy=()):
             "spikes": "+".join("k_sweep<float,%d,%d,true>" % (nt, ct_vw(nt)) for nt in nts),
             "ysweep": "+".join("k_sweep<float,%d,%d,false>" % (nt, ct_y(nt)) for nt in nts),
             "recover": "+".join("k_recover<float,%d,%d>" % (nt, ct_y(nt)) for nt in nts),
-            "residual": "k_residual<double,%d,2>" % tw}
+            "residual": "+".join(dict.fromkeys("k_residual_mm<%d,%d>" % (nt, ncg) if dense(nt) else "k_residual<double,%d,2>" % tw
+                                               for nt in nts))}
 
 
 def main():
@@ -435,7 +439,7 @@ def bench_single(args, torch, hs):
     passes = max(1, eager["last"]["solve_passes"])
     counts = {st: algorithmic_counts(st, n, A.nnz, k, k, nrhs, P_auto, 4) for st in STAGES}
     counts["spikes"] = spike_counts(eager["work"], 4)
-    names = kernel_names_for([mixed["last"]["b"] // 16], nrhs)
+    names = kernel_names_for([mixed["last"]["b"] // 16], nrhs, fill=cfg["fill"])
     stage_roof = stage_roofline(avg, counts, passes, 1, args.config, names)
     roof = roofline_of(stage_roof, avg)
 
@@ -568,7 +572,7 @@ def bench_batch(args, torch, hs):
             counts[st][1] += b
     counts["spikes"] = spike_counts(eager["work"], 4)
     # the b = 64 group of the batch has thousands of partitions: the one-copy factor variant
-    names = kernel_names_for(sorted(nts), C4["nrhs_hi"], one_copy=(4,))
+    names = kernel_names_for(sorted(nts), C4["nrhs_hi"], one_copy=(4,), fill=C4["fill"])
     stage_roof = stage_roofline(avg, counts, passes, groups, "c4", names)
     roof = roofline_of(stage_roof, avg)
 

@@ -1182,7 +1182,7 @@ int Engine::factor() {
                 set_err("zero or non-finite pivot in partition %s%ld", "", (long)q);
                 return SPIKE_ERR_SINGULAR;
             }
-        // a 4x4 panel pivot of the MFMA inversion was zero: redo T_i with full partial pivoting
+        // a pivot of the MFMA inversion was zero among its four rows: redo T_i with full partial pivoting
         // (the whole block in LDS; b = 256 pivots inside 16 x 16 panels already)
         const size_t smem = ((size_t)g.b * g.b + 2 * g.b) * hs;
         if (stv[1] && !g.ifs.empty() && smem <= 160 * 1024) {
