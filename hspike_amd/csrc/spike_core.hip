@@ -396,6 +396,12 @@ int factor_slots(int tcode, int nt) {
 // the per-partition work -- V spikes, tips, interfaces of the reduced system, its sweeps -- is
 // what the partition count buys) uses partitions of 96 blocks; measured on the 4096-system batch
 // (ms per step): 12 blocks 253.5, 24 227.3, 48 214.2, 96 208.8.
+// The wide groups (b = 256; complex FP64 b = 128) keep the same two lengths, though one dominant system
+// alone on the device would run faster on shorter partitions (60001 rows, k = 200, 16 columns, ms per step: 12
+// blocks 8.4, 6 5.6, 3 4.8).  The sweeps of the reduced system then contract less, and a matrix whose spikes decay
+// slowly loses more than that (five-point Laplacian on a grid of width 200, 60000 rows, diagonal 4.05, reduced
+// sweeps: 12 blocks 10, 6 20, 3 50 of the 64 allowed; diagonal 4, on the direct reduced solve, ms per step: 1162,
+// 2254, 4713), as do batches (64 systems of 100000 rows: 12 blocks 132, 6 161, 3 221, and 96 blocks 76).
 extern "C" int spike_autotune_partitions_tuned(int n, int ku, int kl, int nrhs, int dtype, int precision, int tune) {
     (void)nrhs;
     const int NT = block_nt(ku, kl);
@@ -411,11 +417,7 @@ extern "C" int spike_autotune_partitions_tuned(int n, int ku, int kl, int nrhs, 
         const long x = v ? atol(v) : 0;
         return x > 0 ? x : 96L;
     }();
-    long blocks_per_part = tune == SPIKE_TUNE_THROUGHPUT ? bpp_throughput : bpp_latency;
-    // the wide groups take a whole CU per partition and about 0.3 ms per 256-row block: three blocks per
-    // partition (n = 60001, k = 200, 16 columns, ms per step: 12 blocks 9.4, 4 blocks 5.29, 3 blocks
-    // 4.80; 2 blocks 3.94, but the couplings of weakly dominant matrices would then need many sweeps)
-    if (wide_group(type_code(dtype, precision), NT)) blocks_per_part = std::min(blocks_per_part, 3L);
+    const long blocks_per_part = tune == SPIKE_TUNE_THROUGHPUT ? bpp_throughput : bpp_latency;
     const long rows_target = blocks_per_part * b;
     long P = n / rows_target;
     const long slots = factor_slots(type_code(dtype, precision), NT);

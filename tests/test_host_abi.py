@@ -4,6 +4,8 @@ No GPU compute is called here."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -196,6 +198,27 @@ def test_autotuner_is_pure():
     for n, k in ((200_000, 64), (37_000, 4), (1_000, 16)):
         t = hs.autotune_partitions(n, k, k, 4, tune="throughput")
         assert 1 <= t <= hs.autotune_partitions(n, k, k, 4)
+
+
+def test_autotuner_blocks_per_partition():
+    """About 12 blocks per partition (latency) and 96 (throughput) for every block size, the wide groups
+    among them (b = 256; complex FP64 b = 128), where shorter partitions put weakly dominant systems on the
+    direct reduced solve; the environment's values take the place of both."""
+    code = """if 1:
+        import hspike_amd as hs
+        for n, ku, kl, cplx, prec in ((60_001, 200, 200, False, hs.SPIKE_PREC_MIXED), (60_001, 10, 129, False, hs.SPIKE_PREC_FP64),
+                                      (50_000, 256, 3, True, hs.SPIKE_PREC_MIXED), (30_000, 100, 128, True, hs.SPIKE_PREC_FP64),
+                                      (30_000, 64, 40, False, hs.SPIKE_PREC_MIXED), (9_999, 2, 2, False, hs.SPIKE_PREC_FP64)):
+            b = next(x for x in (16, 32, 64, 128, 256) if max(ku, kl) <= x)
+            print(hs.autotune_partitions(n, ku, kl, 4, complex=cplx, precision=prec) == max(1, n // (LAT * b)),
+                  hs.autotune_partitions(n, ku, kl, 4, complex=cplx, precision=prec, tune="throughput") == max(1, n // (THR * b)))
+    """
+    for env, lat, thr in (({}, 12, 96), ({"HSPIKE_BLOCKS_PER_PART": "7", "HSPIKE_BLOCKS_PER_PART_BATCH": "20"}, 7, 20)):
+        e = {k: v for k, v in os.environ.items() if not k.startswith("HSPIKE_BLOCKS")}
+        r = subprocess.run([sys.executable, "-c", code.replace("LAT", str(lat)).replace("THR", str(thr))], cwd=ROOT,
+                           env=dict(e, **env), capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stderr
+        assert r.stdout.split() == ["True"] * 12, (env, r.stdout)
 
 
 # ---------------------------------------------------------------- drop-in boundary (headers, memory ABI)
