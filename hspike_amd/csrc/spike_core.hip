@@ -35,6 +35,7 @@
 #include <initializer_list>
 
 #include "spike_dev.h"
+#include "spike_rules.h"
 #include "spike_kernels.inc"
 #include "spike_kernels_wide.inc"
 #include "spike_kernels_aux.inc"
@@ -741,22 +742,9 @@ void launch_recover(int nitems, hipStream_t s, const SweepItem *items, const Par
                            part_iface, ymax, (const Q4<T> *)wsave, accumulate, active, wstop);
 }
 
-// The residual kernel of a system, from the system and its columns in the chunk alone (a system gets the
-// same bits alone and in a batch).  The dense-tile kernel costs about the same whatever the fill and
-// reads x once per 16 rows, the gather kernel's time follows the nonzeros and the columns.  us per
-// residual, gather / dense tile (real values):
-//   k = 16, 600000 rows, 15% / 50% fill: 4 columns 49 / 47, 70 / 54; 16 columns 116 / 65, 153 / 87
-//   k = 30, 500000 rows: 4 columns 51 / 67, 101 / 81; 16 columns 109 / 78, 170 / 97
-//   k = 64, 400000 rows: 4 columns 60 / 97, 172 / 144; 16 columns 110 / 102, 224 / 157
-//   k = 100, 300000 rows: 16 columns 108 / 155, 251 / 252; 32 columns 204 / 220, 424 / 317; 64 370 / 350, 771 / 440
-// so: b = 16 always; b = 32 and 64 from 9 columns or a third of the band filled; b = 128 from 33 columns,
-// or from 17 with a quarter filled.
+// the residual kernel of a system (complex systems: always the gather kernel)
 bool dense_residual(int dtype, int nt, int n, int64_t nnz, int ku, int kl, int m) {
-    if (dtype != SPIKE_DTYPE_D || nt > 8) return false;
-    const double fill = (double)nnz / ((double)n * (ku + kl + 1));
-    if (nt == 1) return true;
-    if (nt <= 4) return m > 8 || fill >= 1.0 / 3;
-    return m > 32 || (m > 16 && fill >= 0.25);
+    return dtype == SPIKE_DTYPE_D && dense_tile_residual(nt, n, nnz, ku, kl, m);
 }
 
 // FP64 residual with TW column lanes per row: the narrowest of 4, 8, 16 covering the chunk's

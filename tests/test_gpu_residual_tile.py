@@ -50,6 +50,33 @@ def test_reported_residual(hs, n, ku, kl, nrhs):
     t.close()
 
 
+@pytest.mark.parametrize("n,ku,kl,nrhs", [(63, 2, 2, 9), (65, 0, 4, 10), (64, 3, 0, 9), (1, 0, 0, 9), (17, 1, 1, 64)])
+def test_small_orders_with_the_dense_tile(hs, n, ku, kl, nrhs):
+    """More than 8 columns: at b = 16 the dense tile whatever the entries per row."""
+    test_reported_residual(hs, n, ku, kl, nrhs)
+
+
+@pytest.mark.parametrize("k,nrhs", [(7, 1), (7, 4), (7, 16), (30, 3), (30, 9), (61, 8), (61, 16), (61, 33), (128, 17), (128, 64)])
+def test_stencil(hs, k, nrhs):
+    """Five-point Laplacian on a grid of width k, 5 entries per row: both residual kernels, by the columns."""
+    n = 9 * k + 4
+    off = np.array([-k, -1, 0, 1, k])
+    i = np.repeat(np.arange(n), 5)
+    j = i + np.tile(off, n)
+    v = np.tile([-1.0, -1.0, 4.5, -1.0, -1.0], n)
+    keep = (j >= 0) & (j < n)
+    rp = np.zeros(n + 1, dtype=np.int32)
+    np.add.at(rp, i[keep] + 1, 1)
+    A = hs.CSRMatrix(n, np.cumsum(rp).astype(np.int32), j[keep].astype(np.int32), v[keep])
+    B = hs.gen_dense(n, nrhs, seed=4)
+    s = hs.Solver("mixed", max_refine=0, tol=1e-3)
+    s.set_matrix(A)
+    X = s.solve(B)
+    got, ref = s.stats()["max_rel_residual"], cpu_relres(A, X, B).max()
+    assert abs(got - ref) <= 1e-6 * ref + 1e-15
+    s.close()
+
+
 def test_duplicate_entries_are_summed(hs):
     """Entry (r, r) split in two halves: the factorization keeps one of them, the residual sums both, so
     the solve ends unconverged instead of with a wrong answer."""
