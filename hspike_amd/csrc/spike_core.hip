@@ -469,11 +469,12 @@ struct Group {
     std::vector<int> part_iface;
     std::vector<RowChunk> chunks;
     std::vector<int> chunk0;                // per system in the group: first chunk, +1 end
+    std::vector<int> slab_sys;              // systems whose norms are summed in slabs (k_norm_slabs)
     std::vector<SysDev> sysdev;
     std::vector<int> sys_part0;             // global partition of each system
     int64_t nblk = 0;
     int64_t rows_pad = 0;                   // nblk * b
-    DevBuf d_parts, d_ifs, d_part_iface, d_chunks, d_chunk0, d_sysdev, d_active, d_red_active;
+    DevBuf d_parts, d_ifs, d_part_iface, d_chunks, d_chunk0, d_slab_sys, d_sysdev, d_active, d_red_active;
     DevBuf blkmap;                          // partition of each block
     DevBuf D, U, C, R, Bt, Ct;              // factor type
     DevBuf Wf, Vf;                          // forward-swept W spike (all blocks) and V spike (last two blocks)
@@ -912,7 +913,7 @@ int Engine::factor() {
         g.b = 16 * g.NT;
         g.tcode = tcode;
         g.sys = members;
-        g.ifs.clear(); g.part_iface.clear(); g.chunks.clear(); g.chunk0.clear();
+        g.ifs.clear(); g.part_iface.clear(); g.chunks.clear(); g.chunk0.clear(); g.slab_sys.clear();
         g.sys_part0.clear();
         int64_t blk = 0;
         for (int gs = 0; gs < (int)members.size(); ++gs) {
@@ -943,6 +944,7 @@ int Engine::factor() {
             }
             g.chunk0.push_back((int)g.chunks.size());
             for (int r = 0; r < S.n; r += RES_ROWS) g.chunks.push_back({gs, r});
+            if ((int)g.chunks.size() - g.chunk0.back() > NORM_MIN) g.slab_sys.push_back(gs);
             SysDev sd;
             memset(&sd, 0, sizeof sd);
             sd.rowptr = S.d_rowptr; sd.colind = S.d_colind; sd.aij = S.d_aij;
@@ -973,6 +975,7 @@ int Engine::factor() {
             if ((e = upload(g.d_part_iface, g.part_iface.data(), g.part_iface.size() * sizeof(int), s))) return e;
             if ((e = upload(g.d_chunks, g.chunks.data(), g.chunks.size() * sizeof(RowChunk), s))) return e;
             if ((e = upload(g.d_chunk0, g.chunk0.data(), g.chunk0.size() * sizeof(int), s))) return e;
+            if (!g.slab_sys.empty() && (e = upload(g.d_slab_sys, g.slab_sys.data(), g.slab_sys.size() * sizeof(int), s))) return e;
             if ((e = upload(g.d_sysdev, g.sysdev.data(), g.sysdev.size() * sizeof(SysDev), s))) return e;
             if ((e = g.blkmap.ensure(g.nblk * sizeof(int)))) return e;
             hipLaunchKernelGGL(k_blkmap, dim3((unsigned)np), dim3(256), 0, s, g.d_parts.as<PartDesc>(), g.blkmap.as<int>());
@@ -1585,12 +1588,12 @@ std::vector<uint64_t> Engine::graph_key(int ymax) const {
     for (int gi = 0; gi < ngroups; ++gi) {
         const Group &g = *groups[gi];
         k.insert(k.end(), {(uint64_t)g.NT, (uint64_t)g.tcode, (uint64_t)g.ct_y, (uint64_t)g.n_items_y, (uint64_t)g.n_items_r,
-                           (uint64_t)g.ifs.size(), (uint64_t)g.chunks.size(), (uint64_t)g.sys.size(), (uint64_t)g.ymax, (uint64_t)g.res_kernels});
+                           (uint64_t)g.ifs.size(), (uint64_t)g.chunks.size(), (uint64_t)g.sys.size(), (uint64_t)g.ymax, (uint64_t)g.res_kernels, (uint64_t)g.slab_sys.size()});
         const DevBuf *bufs[] = {&g.D, &g.U, &g.C, &g.R, &g.Wf, &g.Vf, &g.wstop, &g.rstop, &g.Bt, &g.Ct, &g.vt, &g.vb, &g.wt, &g.wb, &g.T,
                                 &g.yt, &g.yb, &g.red0, &g.red1, &g.scratch, &g.partials, &g.norms, &g.conv, &g.rwork,
                                 &g.xrm, &g.d_active, &g.d_red_active, &g.d_sysstat, &g.d_direct, &g.d_summary,
                                 &g.items_yb, &g.items_yr, &g.items_rb, &g.items_rr, &g.d_parts, &g.d_ifs, &g.d_part_iface,
-                                &g.d_chunks, &g.d_chunk0, &g.d_sysdev};
+                                &g.d_chunks, &g.d_chunk0, &g.d_slab_sys, &g.d_sysdev};
         for (auto b : bufs) k.push_back((uint64_t)(uintptr_t)b->p);
         k.insert(k.end(), g.solve_key.begin(), g.solve_key.end());
     }
@@ -1780,13 +1783,12 @@ int Engine::run_passes(int ymax, bool capture, double rtol, int max_refine, doub
         for (int gi = 0; gi < ngroups; ++gi) {
             Group &g = *groups[gi];
             const int ngs = (int)g.sys.size();
-            bool slabs = false;
-            for (int gs = 0; gs < ngs; ++gs) slabs |= g.chunk0[gs + 1] - g.chunk0[gs] > NORM_MIN;
-            if (slabs)
-                hipLaunchKernelGGL(k_norm_slabs, dim3((unsigned)ngs * NORM_SLABS), dim3(256), 0, g.st, g.d_chunk0.as<int>(),
-                                   g.partials.as<double>(), ymax);
+            const unsigned nslab = (unsigned)g.slab_sys.size();
+            if (nslab)
+                hipLaunchKernelGGL(k_norm_slabs, dim3(nslab * NORM_SLABS), dim3(256), 0, g.st, (const int *)g.d_slab_sys.p,
+                                   g.d_chunk0.as<int>(), g.partials.as<double>(), ymax);
             hipLaunchKernelGGL(k_norm_reduce, dim3((unsigned)(ngs * ymax)), dim3(256), 0, g.st, g.d_chunk0.as<int>(),
-                               g.d_sysdev.as<SysDev>(), g.partials.as<double>(), g.norms.as<double>(), ymax, slabs ? 1 : 0);
+                               g.d_sysdev.as<SysDev>(), g.partials.as<double>(), g.norms.as<double>(), ymax, nslab ? 1 : 0);
             hipLaunchKernelGGL(k_refine_check, dim3((ngs + 255) / 256), dim3(256), 0, g.st, g.d_sysstat.as<SysStat>(), ngs,
                                (const SysDev *)g.d_sysdev.p, (const double *)g.norms.p, ymax, o.tol, it, max_refine,
                                g.d_active.as<int>());
