@@ -62,3 +62,27 @@ def test_zero_column_is_singular(hs, col):
         hs.band_solve(hs.CSRMatrix(A.n, A.rowptr, A.colind, aij), np.ones((100, 1)))
     assert ex.value.code == -4
     assert "column %d" % col in str(ex.value)
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("n,ku,row", [(200, 0, 70), (200, 3, 70), (64, 0, 0), (300, 40, 256), (130, 100, 127)])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_nonfinite_right_hand_side_stays_where_it_is_coupled(hs, n, ku, row, cplx, value):
+    """Upper triangular bands (kl = 0): the rows below a row with a non-finite right-hand side do not depend on
+    it; on a diagonal matrix no other row does."""
+    rng = np.random.default_rng(3)
+    i = np.repeat(np.arange(n), ku + 1)
+    j = i + np.tile(np.arange(ku + 1), n)
+    keep = j < n
+    v = rng.uniform(-1, 1, i.size) / (ku + 1)
+    v[j == i] = 2.0
+    rp = np.zeros(n + 1, dtype=np.int32)
+    np.add.at(rp, i[keep] + 1, 1)
+    A = hs.CSRMatrix(n, np.cumsum(rp).astype(np.int32), j[keep].astype(np.int32), v[keep] + 0j if cplx else v[keep])
+    B = hs.gen_dense(n, 1, seed=5, complex=cplx)
+    X0, _ = hs.band_solve(A, B)
+    B[row] = value
+    X, _ = hs.band_solve(A, B)
+    assert not np.isfinite(X[row]).any()
+    free = np.arange(n) > row if ku else np.arange(n) != row
+    assert np.allclose(X[free], X0[free], rtol=1e-13, atol=1e-13)
