@@ -36,3 +36,31 @@ def test_items_stop_apart(oracle_mod, prec, k, cplx, nparts):
         Xo = oracle_mod.direct_solve(oracle_mod.CSR(n, A.rowptr, A.colind, aij), B)
         assert np.linalg.norm(X - Xo) / np.linalg.norm(Xo) <= 1e-11, trial
     s.close()
+
+
+@pytest.mark.parametrize("prec,ku", [("mixed", 2), ("mixed", 60), ("mixed", 140), ("fp64", 2), ("fp64", 140)])
+def test_overflowing_spike_is_not_taken_for_a_decayed_one(prec, ku):
+    """Two chains in one matrix, even and odd rows: the even W column grows until it overflows in block 2 and is
+    NaN from there on, the odd one decays to zero.  The bottom tip of the even column must not be finite (a
+    maximum that drops NaN ends the chain there and leaves a tip of zeros)."""
+    import hspike_amd as hs
+    hs.load()
+    b = next(x for x in (16, 32, 64, 128, 256) if ku <= x)
+    n = 2 * 7 * b
+    g = (1e13 if prec == "mixed" else 1e110) ** (2.0 / b)
+    i = np.arange(2, n)
+    rows = np.concatenate([np.arange(n), i, [0]])
+    cols = np.concatenate([np.arange(n), i - 2, [ku]])
+    vals = np.concatenate([np.ones(n), np.where(i % 2 == 0, -g, -0.5), [1e-30]])
+    order = np.lexsort((cols, rows))
+    rp = np.zeros(n + 1, dtype=np.int32)
+    np.add.at(rp, rows + 1, 1)
+    A = hs.CSRMatrix(n, np.cumsum(rp).astype(np.int32), cols[order].astype(np.int32), vals[order])
+    B = np.zeros((n, 1))
+    B[1] = 1.0
+    s = hs.Solver(prec, partitions=2, max_refine=0, reduced_solver="jacobi")
+    s.set_matrix(A)
+    s.solve(B, allow_unconverged=True)
+    Wb = s.tips()["Wb"][1]
+    assert s.stats()["b"] == b and not np.isfinite(Wb[:, 0]).any(), Wb
+    s.close()
