@@ -150,6 +150,12 @@ template <typename T> __device__ __forceinline__ int acol(int c) {
     return row_major_groups<T>() ? c : ((c & ~15) | ((c & 3) << 2) | ((c >> 2) & 3));
 }
 template <typename T> struct alignas(4 * sizeof(T)) Q4 { T v[4]; };
+// four adjacent values of a padded LDS row: such rows are aligned to 16 bytes, not to a Q4 of 8- and 16-byte types
+template <typename T> __device__ __forceinline__ Q4<T> q4_lds(const T *p) {
+    Q4<T> q;
+    __builtin_memcpy(&q, __builtin_assume_aligned(p, 16), sizeof q);
+    return q;
+}
 
 // 16 x 16 accumulator tile distributed over a wave64 (4 elements per lane)
 template <typename T, bool C = tr<T>::C> struct Tile;
