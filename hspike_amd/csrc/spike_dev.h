@@ -213,9 +213,6 @@ template <typename T, int N> __device__ __forceinline__ void tiles_settle(Tile<T
         asm volatile("s_nop 7\n\ts_nop 7" : "+a"(x[0].v), "+a"(x[1].v), "+a"(x[2].v));
     } else if constexpr (!tr<T>::C && N == 4) {
         asm volatile("s_nop 7\n\ts_nop 7" : "+a"(x[0].v), "+a"(x[1].v), "+a"(x[2].v), "+a"(x[3].v));
-    } else if constexpr (!tr<T>::C && N == 8) {
-        asm volatile("s_nop 7\n\ts_nop 7" : "+a"(x[0].v), "+a"(x[1].v), "+a"(x[2].v), "+a"(x[3].v), "+a"(x[4].v),
-                     "+a"(x[5].v), "+a"(x[6].v), "+a"(x[7].v));
     } else if constexpr (tr<T>::C && N == 2) {
         asm volatile("s_nop 7\n\ts_nop 7" : "+a"(x[0].re), "+a"(x[0].im), "+a"(x[1].re), "+a"(x[1].im));
     } else if constexpr (tr<T>::C && N == 4) {
