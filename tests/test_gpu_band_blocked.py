@@ -1,7 +1,8 @@
 """The blocked band LU and the register-window band solves (k_gbtrf_blk, k_gbtrs_fwd / _bwd) through
 spike_band_solve_host: orders around the panel width (32, complex 16) and the 64-row windows, one-sided
-and empty bands, bandwidths at the edges of the register windows, interchanges over the whole lower
-band, and a band too wide for the blocked kernels (kl > 448), which the column kernels take.
+and empty bands, bandwidths at the edges of the register windows, interchanges with rows min(ku, kl) away
+and, by the cyclic matrices, with the last row of the lower band, and a band too wide for the blocked
+kernels (kl > 448), which the column kernels take.
 
 The matrices have singular values >= 1.2 and norms <= 2.8 (a permutation of 2 I inside the band plus
 noise with row sums <= 0.8), so after the FP64 refinement the residual is at rounding level: 1e-14,
@@ -19,8 +20,9 @@ def hs():
     return hspike_amd
 
 
-def pivoting_band(hs, n, ku, kl, seed, cplx):
-    """2 at (i, s(i)), s reversing groups of min(ku, kl) + 1 rows; zero diagonal where s(i) != i."""
+def pivoting_band(hs, n, ku, kl, seed, cplx, cyclic=False):
+    """2 at (i, s(i)), zero diagonal where s(i) != i; s reverses groups of min(ku, kl) + 1 rows, or, cyclic,
+    moves each row of groups of kl + 1 one column up and the group's last row to its first column."""
     rng = np.random.default_rng(seed)
     i = np.repeat(np.arange(n), ku + kl + 1)
     j = i + np.tile(np.arange(-kl, ku + 1), n)
@@ -29,9 +31,9 @@ def pivoting_band(hs, n, ku, kl, seed, cplx):
     v = rng.uniform(-1, 1, i.size) * (0.8 / max(ku + kl, 1))
     if cplx:
         v = v * np.exp(2j * np.pi * rng.uniform(0, 1, i.size))
-    m = min(ku, kl) + 1
+    m = kl + 1 if cyclic else min(ku, kl) + 1
     first = (i // m) * m
-    to = np.where(first + m <= n, 2 * first + m - 1 - i, i)
+    to = np.where(first + m <= n, np.where(i + 1 < first + m, i + 1, first) if cyclic else 2 * first + m - 1 - i, i)
     v[(j == i) & (to != i)] = 0.0
     v[j == to] = 2.0
     rp = np.zeros(n + 1, dtype=np.int32)
@@ -47,6 +49,21 @@ def pivoting_band(hs, n, ku, kl, seed, cplx):
 ])
 def test_band_solve_matches_oracle(hs, oracle_mod, n, ku, kl, nrhs, cplx):
     A = pivoting_band(hs, n, ku, kl, seed=n + ku, cplx=cplx)
+    B = hs.gen_dense(n, nrhs, seed=3, complex=cplx)
+    X, rel = hs.band_solve(A, B)
+    assert rel.max() <= 1e-14, rel
+    Xo = oracle_mod.direct_solve(oracle_mod.CSR(A.n, A.rowptr, A.colind, A.aij), B)
+    assert np.linalg.norm(X - Xo) / np.linalg.norm(Xo) <= 1e-12
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("n,ku,kl,nrhs", [
+    (2, 1, 1, 1), (33, 2, 7, 1), (65, 16, 31, 2), (97, 1, 32, 1), (200, 64, 64, 3), (300, 65, 100, 1), (700, 100, 191, 3), (1000, 1, 192, 1),
+    (1400, 20, 448, 1), (1400, 10, 460, 2),
+])
+def test_interchanges_with_the_last_row_of_the_band(hs, oracle_mod, n, ku, kl, nrhs, cplx):
+    A = pivoting_band(hs, n, ku, kl, seed=n + kl, cplx=cplx, cyclic=True)
+    assert (A.rowptr[1:] > A.rowptr[:-1]).all() and abs(A.aij[(A.colind == 0) & (np.repeat(np.arange(n), np.diff(A.rowptr)) == kl)]) == 2.0
     B = hs.gen_dense(n, nrhs, seed=3, complex=cplx)
     X, rel = hs.band_solve(A, B)
     assert rel.max() <= 1e-14, rel

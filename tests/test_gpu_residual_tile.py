@@ -1,7 +1,8 @@
 """The dense-tile residual (k_residual_mm) through whole solves: orders around its 64-row chunks and
-16-row tiles, one-sided bands, one to four column tiles with odd counts, empty rows off the diagonal,
-rows stored in any column order and split entries (duplicates are summed), in a batch that mixes
-systems of both residual kernels.
+16-row tiles (test_small_orders_with_the_dense_tile where few columns leave them to the gather kernel),
+one-sided bands, one to four column tiles with odd counts, rows stored in any column order and split
+entries (duplicates are summed), bands with five entries per row, in a batch that mixes systems of both
+residual kernels.
 
 The solver's reported residual against a CPU residual (numpy, FP64) of the returned solution: both
 are rounding-level quantities of the same solution, so they are compared on a solve stopped after its

@@ -1,7 +1,7 @@
 """The wide factor (b = 256, and complex FP64 at b = 128): pivot tiles that are dominant by rows (the
 in-register inversion), tiles that need interchanges over all 16 rows (the LDS one), and mixes of both
-in one matrix; unequal bandwidths, so tiles without entries of B_j and C_j are skipped; one-row last
-blocks.
+in one matrix; unequal bandwidths, so tiles without entries of B_j and C_j are skipped; last blocks of
+16 and 17 rows, of one row, and whole ones.
 
 The matrices are a permutation of 2 I inside 16-row groups (or 2 I) plus band noise with row sums at
 most 0.8: singular values are at least 1.2, so against the oracle's band LU the FP64 solution differs
@@ -41,9 +41,10 @@ def reversed_band(hs, n, ku, kl, group, rows_from, cplx, seed):
 @pytest.mark.parametrize("ku,kl,prec,cplx", [(200, 140, "mixed", False), (130, 256, "mixed", False), (150, 190, "fp64", False),
                                              (140, 160, "mixed", True), (100, 128, "fp64", True)])
 @pytest.mark.parametrize("group,frac", [(1, 1.0), (16, 0.0), (16, 0.5)])
-def test_wide_factor_matches_oracle(hs, oracle_mod, ku, kl, prec, cplx, group, frac):
+@pytest.mark.parametrize("rest", [16, 0])
+def test_wide_factor_matches_oracle(hs, oracle_mod, ku, kl, prec, cplx, group, frac, rest):
     b = 128 if max(ku, kl) <= 128 else 256
-    part = 2 * b + 16                            # partitions start on multiples of 16
+    part = 2 * b + rest                          # partitions start on multiples of 16, the last has one row more
     n = 2 * part + 1
     A = reversed_band(hs, n, ku, kl, group, int(frac * n) // 16 * 16, cplx, seed=ku)
     B = hs.gen_dense(n, 2, seed=5, complex=cplx)
