@@ -39,7 +39,7 @@ def test_reduced_solution_matches_oracle(hs, oracle_mod, ku, kl, P, nrhs):
     s.close()
 
 
-@pytest.mark.parametrize("k,P,nrhs", [(3, 3, 1), (20, 4, 17), (40, 3, 5), (90, 2, 20), (140, 2, 3)])
+@pytest.mark.parametrize("k,P,nrhs", [(3, 3, 1), (3, 4, 33), (20, 4, 17), (20, 3, 40), (30, 4, 64), (40, 3, 5), (40, 2, 33), (90, 2, 20), (140, 2, 3)])
 def test_complex_reduced(hs, oracle_mod, k, P, nrhs):
     b = next(x for x in (16, 32, 64, 128, 256) if k <= x)
     n = P * (2 * b + 5) + 3
