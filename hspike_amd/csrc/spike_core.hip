@@ -1217,17 +1217,19 @@ int Engine::factor() {
 }
 
 // ============================================================================ direct reduced solve
-// Band LU of nd systems whose lower bandwidth is at most klmax: blocked where its LDS holds the
-// multipliers, else column by column (lds: that kernel's dynamic LDS).
+// Band LU of nd systems (bs: their descriptors on the host), each by its own kernel; lds: k_gbtrf's dynamic LDS
 template <typename H>
-int launch_gbtrf(int nd, int klmax, size_t lds, hipStream_t s, const BandSys *sys, H *ab, int *piv, int *info) {
-    if (klmax <= GB_KL_MAX) {
-        const size_t need = gb_blk_lds<H>(klmax);
-        HIPCK(hipFuncSetAttribute((const void *)k_gbtrf_blk<H>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gb_blk_lds<H>(GB_KL_MAX)));
-        hipLaunchKernelGGL(k_gbtrf_blk<H>, dim3(nd), dim3(GB_BTHREADS), need, s, sys, ab, piv, info);
-    } else {
-        hipLaunchKernelGGL(k_gbtrf<H>, dim3(nd), dim3(GB_THREADS), lds, s, sys, ab, piv, info);
+int launch_gbtrf(const BandSys *bs, int nd, size_t lds, hipStream_t s, const BandSys *sys, H *ab, int *piv, int *info) {
+    int klmax = -1, columns = 0;
+    for (int q = 0; q < nd; ++q) {
+        if (bs[q].panels) klmax = std::max(klmax, bs[q].kl);
+        else ++columns;
     }
+    if (klmax >= 0) {
+        HIPCK(hipFuncSetAttribute((const void *)k_gbtrf_blk<H>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gb_blk_lds<H>(GB_KL_MAX)));
+        hipLaunchKernelGGL(k_gbtrf_blk<H>, dim3(nd), dim3(GB_BTHREADS), gb_blk_lds<H>(klmax), s, sys, ab, piv, info);
+    }
+    if (columns) hipLaunchKernelGGL(k_gbtrf<H>, dim3(nd), dim3(GB_THREADS), lds, s, sys, ab, piv, info);
     HIPCK(hipGetLastError());
     return SPIKE_SUCCESS;
 }
@@ -1278,7 +1280,7 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
         g.rd_bs.assign(nd, BandSys{});
         g.rd_desc_h.assign(nd, RedDirect{});
         int64_t ab = 0, pv = 0;
-        int maxP = 1, klmax = 0;
+        int maxP = 1;
         size_t lds = 0;
         for (int q = 0; q < nd; ++q) {
             const SysHost &S = sys[g.sys[g.rd_sys[q]]];
@@ -1287,6 +1289,7 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
             BandSys &B = g.rd_bs[q];
             B.n = S.P * (S.ku + S.kl);
             B.kl = klr; B.ku = kur; B.ldab = 2 * klr + kur + 1;
+            B.panels = band_lu_panels(dtype == SPIKE_DTYPE_Z, klr, kur) ? 1 : 0;
             B.ab = ab; B.piv = pv;
             ab += (int64_t)B.n * B.ldab;
             pv += B.n;
@@ -1295,7 +1298,6 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
             D.iface0 = g.part_iface[D.part0];
             D.P = S.P; D.ku = S.ku; D.kl = S.kl; D.band = q;
             maxP = std::max(maxP, S.P);
-            klmax = std::max(klmax, klr);
             lds = std::max(lds, (size_t)(std::max(klr, 1) + klr + kur + 1) * hs);
         }
         if (lds > 64 * 1024) {
@@ -1314,14 +1316,14 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
             hipLaunchKernelGGL(k_red_band<zd>, dim3(maxP, nd), dim3(256), 0, s, g.rd_desc.as<RedDirect>(), g.rd_bsd.as<BandSys>(),
                                (const zd *)g.vt.p, (const zd *)g.vb.p, (const zd *)g.wt.p, (const zd *)g.wb.p, g.b,
                                g.rd_ab.as<zd>());
-            if ((e = launch_gbtrf<zd>(nd, klmax, lds, s, g.rd_bsd.as<BandSys>(), g.rd_ab.as<zd>(), g.rd_piv.as<int>(),
+            if ((e = launch_gbtrf<zd>(g.rd_bs.data(), nd, lds, s, g.rd_bsd.as<BandSys>(), g.rd_ab.as<zd>(), g.rd_piv.as<int>(),
                                       g.rd_info.as<int>())))
                 return e;
         } else {
             hipLaunchKernelGGL(k_red_band<double>, dim3(maxP, nd), dim3(256), 0, s, g.rd_desc.as<RedDirect>(),
                                g.rd_bsd.as<BandSys>(), (const double *)g.vt.p, (const double *)g.vb.p,
                                (const double *)g.wt.p, (const double *)g.wb.p, g.b, g.rd_ab.as<double>());
-            if ((e = launch_gbtrf<double>(nd, klmax, lds, s, g.rd_bsd.as<BandSys>(), g.rd_ab.as<double>(),
+            if ((e = launch_gbtrf<double>(g.rd_bs.data(), nd, lds, s, g.rd_bsd.as<BandSys>(), g.rd_ab.as<double>(),
                                           g.rd_piv.as<int>(), g.rd_info.as<int>())))
                 return e;
         }
@@ -1338,16 +1340,13 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
     // right-hand sides of this pass for the systems in `which`, band solve, scatter into the iterate
     int64_t xe = 0;
     int maxnr = 1, nrow = 0;
-    std::vector<int> items;
-    std::vector<int> items_g;
+    std::vector<int> items_w;                        // one wave per column (launch_trs_waves)
+    std::vector<int> items;                          // k_gbtrs, panel in LDS
+    std::vector<int> items_g;                        // k_gbtrs, panel in global memory
     std::vector<RedDirect> pass;
     const size_t lds_cap = 48 * 1024;
     size_t lds = 0;
-    int klm = 0, kvm = 0;
-    for (const BandSys &B : g.rd_bs) { klm = std::max(klm, B.kl); kvm = std::max(kvm, B.kl + B.ku); }
-    const int sf = dtype == SPIKE_DTYPE_Z ? trs_slots<zd>(klm) : trs_slots<double>(klm);
-    const int sb = dtype == SPIKE_DTYPE_Z ? trs_slots<zd>(kvm) : trs_slots<double>(kvm);
-    const bool waves = sf && sb;
+    int sf = 0, sb = 0;                              // register slots of the widest system on waves
     for (int q = 0; q < nd; ++q) {
         if (std::find(which.begin(), which.end(), g.rd_sys[q]) == which.end()) continue;
         pass.push_back(g.rd_desc_h[q]);
@@ -1357,8 +1356,12 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
         maxnr = std::max(maxnr, B.n);
         nrow = std::max(nrow, (g.rd_desc_h[q].P - 1) * (g.rd_desc_h[q].ku + g.rd_desc_h[q].kl) * ymax);
         const size_t per_col = (size_t)B.n * hs;
-        if (waves) {
-            for (int c = 0; c < ymax; ++c) items.insert(items.end(), {q, c, 1});
+        const int qf = dtype == SPIKE_DTYPE_Z ? trs_slots<zd>(B.kl) : trs_slots<double>(B.kl);
+        const int qb = dtype == SPIKE_DTYPE_Z ? trs_slots<zd>(B.kl + B.ku) : trs_slots<double>(B.kl + B.ku);
+        if (qf && qb) {
+            sf = std::max(sf, qf);
+            sb = std::max(sb, qb);
+            for (int c = 0; c < ymax; ++c) items_w.insert(items_w.end(), {q, c, 1});
         } else if (per_col <= lds_cap) {
             const int mc = (int)std::min<size_t>({64, (size_t)ymax, lds_cap / per_col});
             for (int c = 0; c < ymax; c += mc) items.insert(items.end(), {q, c, std::min(mc, ymax - c)});
@@ -1373,23 +1376,24 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
     if ((e = upload(g.rd_bsd, g.rd_bs.data(), nd * sizeof(BandSys), s)) ||
         (e = upload(g.rd_pass, pass.data(), npass * sizeof(RedDirect), s)))
         return e;
-    std::vector<int> all(items);
+    std::vector<int> all(items_w);
+    all.insert(all.end(), items.begin(), items.end());
     all.insert(all.end(), items_g.begin(), items_g.end());
     if ((e = upload(g.rd_items, all.data(), all.size() * sizeof(int), s))) return e;
     const unsigned rgrid = (unsigned)std::min<int64_t>(((int64_t)maxnr * ymax + 255) / 256, 4096);
     const unsigned sgrid = (unsigned)std::min<int64_t>(((int64_t)nrow + 255) / 256 + 1, 4096);
-    const int ni = (int)items.size() / 3, ng = (int)items_g.size() / 3;
+    const int nw = (int)items_w.size() / 3, ni = (int)items.size() / 3, ng = (int)items_g.size() / 3;
     if (dtype == SPIKE_DTYPE_Z) {
         hipLaunchKernelGGL(k_red_rhs<zd>, dim3(rgrid, npass), dim3(256), 0, s, g.rd_pass.as<RedDirect>(), g.rd_bsd.as<BandSys>(),
                            (const zd *)g.yt.p, (const zd *)g.yb.p, g.b, ymax, g.rd_x.as<zd>());
-        if (waves) {
-            if ((e = launch_trs_waves<zd>(ni, sf, sb, s, g.rd_bsd.as<BandSys>(), g.rd_items.as<int>(), (const zd *)g.rd_ab.p,
-                                          (const int *)g.rd_piv.p, g.rd_x.as<zd>())))
-                return e;
-        } else if (ni) hipLaunchKernelGGL((k_gbtrs<zd, true>), dim3(ni), dim3(256), lds, s, g.rd_bsd.as<BandSys>(), g.rd_items.as<int>(),
-                                   (const zd *)g.rd_ab.p, (const int *)g.rd_piv.p, g.rd_x.as<zd>());
+        if (nw && (e = launch_trs_waves<zd>(nw, sf, sb, s, g.rd_bsd.as<BandSys>(), g.rd_items.as<int>(),
+                                            (const zd *)g.rd_ab.p, (const int *)g.rd_piv.p, g.rd_x.as<zd>())))
+            return e;
+        if (ni) hipLaunchKernelGGL((k_gbtrs<zd, true>), dim3(ni), dim3(256), lds, s, g.rd_bsd.as<BandSys>(),
+                                   g.rd_items.as<int>() + 3 * nw, (const zd *)g.rd_ab.p, (const int *)g.rd_piv.p,
+                                   g.rd_x.as<zd>());
         if (ng) hipLaunchKernelGGL((k_gbtrs<zd, false>), dim3(ng), dim3(256), 0, s, g.rd_bsd.as<BandSys>(),
-                                   g.rd_items.as<int>() + 3 * ni, (const zd *)g.rd_ab.p, (const int *)g.rd_piv.p,
+                                   g.rd_items.as<int>() + 3 * (nw + ni), (const zd *)g.rd_ab.p, (const int *)g.rd_piv.p,
                                    g.rd_x.as<zd>());
         hipLaunchKernelGGL(k_red_scatter<zd>, dim3(sgrid, npass), dim3(256), 0, s, g.rd_pass.as<RedDirect>(),
                            g.rd_bsd.as<BandSys>(), (const zd *)g.rd_x.p, g.b, ymax, xo.as<zd>());
@@ -1397,15 +1401,14 @@ int Engine::reduced_direct(Group &g, const std::vector<int> &which, DevBuf &xo, 
         hipLaunchKernelGGL(k_red_rhs<double>, dim3(rgrid, npass), dim3(256), 0, s, g.rd_pass.as<RedDirect>(),
                            g.rd_bsd.as<BandSys>(), (const double *)g.yt.p, (const double *)g.yb.p, g.b, ymax,
                            g.rd_x.as<double>());
-        if (waves) {
-            if ((e = launch_trs_waves<double>(ni, sf, sb, s, g.rd_bsd.as<BandSys>(), g.rd_items.as<int>(),
-                                              (const double *)g.rd_ab.p, (const int *)g.rd_piv.p, g.rd_x.as<double>())))
-                return e;
-        } else if (ni) hipLaunchKernelGGL((k_gbtrs<double, true>), dim3(ni), dim3(256), lds, s, g.rd_bsd.as<BandSys>(),
-                                   g.rd_items.as<int>(), (const double *)g.rd_ab.p, (const int *)g.rd_piv.p,
+        if (nw && (e = launch_trs_waves<double>(nw, sf, sb, s, g.rd_bsd.as<BandSys>(), g.rd_items.as<int>(),
+                                                (const double *)g.rd_ab.p, (const int *)g.rd_piv.p, g.rd_x.as<double>())))
+            return e;
+        if (ni) hipLaunchKernelGGL((k_gbtrs<double, true>), dim3(ni), dim3(256), lds, s, g.rd_bsd.as<BandSys>(),
+                                   g.rd_items.as<int>() + 3 * nw, (const double *)g.rd_ab.p, (const int *)g.rd_piv.p,
                                    g.rd_x.as<double>());
         if (ng) hipLaunchKernelGGL((k_gbtrs<double, false>), dim3(ng), dim3(256), 0, s, g.rd_bsd.as<BandSys>(),
-                                   g.rd_items.as<int>() + 3 * ni, (const double *)g.rd_ab.p, (const int *)g.rd_piv.p,
+                                   g.rd_items.as<int>() + 3 * (nw + ni), (const double *)g.rd_ab.p, (const int *)g.rd_piv.p,
                                    g.rd_x.as<double>());
         hipLaunchKernelGGL(k_red_scatter<double>, dim3(sgrid, npass), dim3(256), 0, s, g.rd_pass.as<RedDirect>(),
                            g.rd_bsd.as<BandSys>(), (const double *)g.rd_x.p, g.b, ymax, xo.as<double>());
@@ -2500,6 +2503,7 @@ int band_run(int dtype, int n, int ku, int kl, const int *rowptr, const int *col
     }
     BandSys B{};
     B.n = n; B.kl = kl; B.ku = ku; B.ldab = ldab;
+    B.panels = band_lu_panels(dtype == SPIKE_DTYPE_Z, kl, ku) ? 1 : 0;
     const size_t elems = (size_t)n * ldab;
     const unsigned rg = (unsigned)((n + 255) / 256), fg = (unsigned)std::min<size_t>((elems + 255) / 256, 65536);
     hipLaunchKernelGGL(k_put<BandSys>, dim3(1), dim3(64), 0, st, w.sys, B);
@@ -2510,12 +2514,12 @@ int band_run(int dtype, int n, int ku, int kl, const int *rowptr, const int *col
         hipLaunchKernelGGL(k_fill<zd>, dim3(fg), dim3(256), 0, st, (zd *)w.ab, (int64_t)elems, s_zero_host<zd>());
         hipLaunchKernelGGL(k_csr_to_band<zd>, dim3(rg), dim3(256), 0, st, rowptr, colind, (const zd *)aij, n, kl, ku, ldab,
                            (zd *)w.ab);
-        if (int e = launch_gbtrf<zd>(1, kl, lds_f, st, (const BandSys *)w.sys, (zd *)w.ab, w.piv, w.flags + 3)) return e;
+        if (int e = launch_gbtrf<zd>(&B, 1, lds_f, st, (const BandSys *)w.sys, (zd *)w.ab, w.piv, w.flags + 3)) return e;
     } else {
         hipLaunchKernelGGL(k_fill<double>, dim3(fg), dim3(256), 0, st, (double *)w.ab, (int64_t)elems, 0.0);
         hipLaunchKernelGGL(k_csr_to_band<double>, dim3(rg), dim3(256), 0, st, rowptr, colind, (const double *)aij, n, kl, ku,
                            ldab, (double *)w.ab);
-        if (int e = launch_gbtrf<double>(1, kl, lds_f, st, (const BandSys *)w.sys, (double *)w.ab, w.piv, w.flags + 3)) return e;
+        if (int e = launch_gbtrf<double>(&B, 1, lds_f, st, (const BandSys *)w.sys, (double *)w.ab, w.piv, w.flags + 3)) return e;
     }
     HIPCK(hipGetLastError());
     int info = 0;

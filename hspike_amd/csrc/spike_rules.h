@@ -1,5 +1,6 @@
-// spike_rules.h -- choices between two kernels that depend on a system's sizes alone: plain C++, so that
-// a host compiler builds them too (the tests hold them against measured times of both kernels).
+// spike_rules.h -- choices between two kernels that depend on a system's sizes alone (so a system gets the
+// same bits alone and in a batch): plain C++, so that a host compiler builds them too (the tests hold them
+// against measured times of both kernels).
 #pragma once
 #include <cstdint>
 
@@ -27,3 +28,8 @@ inline bool dense_tile_residual(int nt, int n, int64_t nnz, int ku, int kl, int 
     default: return false;                      // b = 256: the tile does not fit the LDS
     }
 }
+
+// Band LU of one system: true for k_gbtrf_blk (panels), false for k_gbtrf (column by column): the panels' LDS
+// holds the multipliers up to this kl.
+constexpr int BAND_PANEL_KL_MAX = 448;
+inline bool band_lu_panels(bool, int kl, int) { return kl <= BAND_PANEL_KL_MAX; }

@@ -190,3 +190,43 @@ def test_jacobi_only_reports_not_converged_on_nondominant(hs, oracle_mod):
     with pytest.raises(hs.SpikeError) as ex:
         s.solve(B)
     assert ex.value.code == -5
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+def test_direct_batch_equals_alone(hs, cplx):
+    """Reduced systems solved directly in one batch, with bandwidths on both sides of what the panel LU and the
+    register-window solves take: each system has the bits it has alone."""
+    import ctypes
+    import torch
+    from hspike_amd import _lib
+    dev = torch.device("cuda:0")
+
+    def batch():
+        bt = hs.Batch("fp64", partitions=2)
+        bt.close()
+        opts = _lib.default_opts(precision=hs.SPIKE_PREC_FP64, tol=1e-10, max_refine=0, partitions=2, reduced_solver=hs.SPIKE_RED_DIRECT)
+        h = ctypes.c_void_p()
+        _lib.check(bt._L.spike_batch_create(ctypes.byref(h), ctypes.byref(opts)), "spike_batch_create")
+        bt._h = h
+        return bt
+
+    systems = []
+    for i, k in enumerate([130, 200, 145] if not cplx else [20, 64, 40, 130, 200]):
+        b = 256 if k > 128 else 64
+        n = 2 * (2 * b + 30) + i
+        A = hs.gen_banded(n, k, k, fill=0.5, dom=(1.1, 1.1), diag_floor=1.0, seed=i, complex=cplx)
+        B = hs.gen_dense(n, 2, seed=7 + i, complex=cplx)
+        d = dict(n=n, nrhs=2, rowptr=torch.from_numpy(A.rowptr).to(dev), colind=torch.from_numpy(A.colind).to(dev),
+                 aij=torch.from_numpy(A.aij).to(dev), b=torch.from_numpy(np.ascontiguousarray(B.T)).to(dev))
+        systems.append(dict(d, x=torch.zeros_like(d["b"])))
+    bt = batch()
+    rel, _ = bt.solve_dev(systems, complex=cplx)
+    assert rel.max() <= 1e-10
+    for s in systems:
+        alone = dict(s, x=torch.zeros_like(s["x"]))
+        b1 = batch()
+        b1.solve_dev([alone], complex=cplx)
+        torch.cuda.synchronize()
+        assert torch.equal(alone["x"], s["x"]), s["n"]
+        b1.close()
+    bt.close()
