@@ -29,7 +29,14 @@ inline bool dense_tile_residual(int nt, int n, int64_t nnz, int ku, int kl, int 
     }
 }
 
-// Band LU of one system: true for k_gbtrf_blk (panels), false for k_gbtrf (column by column): the panels' LDS
-// holds the multipliers up to this kl.
+// Band LU of one system: true for k_gbtrf_blk (panels), false for k_gbtrf (column by column).  Real bands take
+// the panels wherever their LDS holds the multipliers.  Complex panels are half as wide and pay more per row of
+// kl, so narrow bands and those with few superdiagonals stay with the columns.  us for 1000 columns, columns /
+// panels, complex (kl, ku): (1, 1) 1950 / 3360, (64, 64) 3472 / 4013, (90, 90) 4618 / 4556, (100, 100) 5114 / 4942,
+// (200, 200) 12598 / 7113, (60, 200) 5192 / 4665, (200, 60) 5572 / 6416, (400, 5) 7705 / 10422, (30, 448) 5400 / 4495;
+// real: (1, 1) 1597 / 1271, (100, 100) 4557 / 1844, (400, 5) 11318 / 3235.
 constexpr int BAND_PANEL_KL_MAX = 448;
-inline bool band_lu_panels(bool, int kl, int) { return kl <= BAND_PANEL_KL_MAX; }
+inline bool band_lu_panels(bool cplx, int kl, int ku) {
+    if (kl > BAND_PANEL_KL_MAX) return false;
+    return !cplx || 3e-4 * kl * ku >= 1.6 + 0.01 * kl + 0.003 * ku;
+}

@@ -1,8 +1,8 @@
 """The blocked band LU and the register-window band solves (k_gbtrf_blk, k_gbtrs_fwd / _bwd) through
 spike_band_solve_host: orders around the panel width (32, complex 16) and the 64-row windows, one-sided
 and empty bands, bandwidths at the edges of the register windows, interchanges with rows min(ku, kl) away
-and, by the cyclic matrices, with the last row of the lower band, and a band too wide for the blocked
-kernels (kl > 448), which the column kernels take.
+and, by the cyclic matrices, with the last row of the lower band, complex bands on both sides of the line
+between panels and columns (band_lu_panels), and a band too wide for the panels (kl > 448).
 
 The matrices have singular values >= 1.2 and norms <= 2.8 (a permutation of 2 I inside the band plus
 noise with row sums <= 0.8), so after the FP64 refinement the residual is at rounding level: 1e-14,
@@ -69,6 +69,13 @@ def test_interchanges_with_the_last_row_of_the_band(hs, oracle_mod, n, ku, kl, n
     assert rel.max() <= 1e-14, rel
     Xo = oracle_mod.direct_solve(oracle_mod.CSR(A.n, A.rowptr, A.colind, A.aij), B)
     assert np.linalg.norm(X - Xo) / np.linalg.norm(Xo) <= 1e-12
+
+
+@pytest.mark.parametrize("n,ku,kl,nrhs", [(112, 100, 110, 1), (113, 112, 100, 2), (127, 110, 110, 1), (129, 120, 128, 3), (300, 100, 95, 1),
+                                          (300, 95, 90, 1), (700, 448, 31, 1), (640, 300, 448, 1)])
+def test_complex_panels(hs, oracle_mod, n, ku, kl, nrhs):
+    test_band_solve_matches_oracle(hs, oracle_mod, n, ku, kl, nrhs, True)
+    test_interchanges_with_the_last_row_of_the_band(hs, oracle_mod, n, ku, min(kl, n - 1), nrhs, True)
 
 
 @pytest.mark.parametrize("col", [0, 31, 32, 77, 99])
