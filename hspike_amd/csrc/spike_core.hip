@@ -422,7 +422,7 @@ extern "C" int spike_autotune_partitions_tuned(int n, int ku, int kl, int nrhs, 
     const long rows_target = blocks_per_part * b;
     long P = n / rows_target;
     const long slots = factor_slots(type_code(dtype, precision), NT);
-    if (slots > 0) P = std::min(P, slots);
+    if (slots > 0 && P > slots) P = capped_partitions(n, slots, b);
     const long min_rows = std::max(2 * b, ku + kl);
     P = std::min(P, (long)n / std::max(1L, min_rows));
     P = std::max(1L, std::min(P, 8192L));

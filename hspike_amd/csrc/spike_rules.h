@@ -40,3 +40,17 @@ inline bool band_lu_panels(bool cplx, int kl, int ku) {
     if (kl > BAND_PANEL_KL_MAX) return false;
     return !cplx || 3e-4 * kl * ku >= 1.6 + 0.01 * kl + 0.003 * ku;
 }
+
+// Partition count where the device's factor workgroups (`slots`) cap it.  Every partition has n / P rows and the
+// last one the remainder too, up to P - 1 rows: with thousands of short partitions that is a chain many times
+// the others' (10^6 rows on 3072 partitions: 121 blocks of 16 rows behind 3071 chains of 21; one column 424 us per
+// FP64 solve, 285 on 3584 partitions, whose last chain has 22).  If the remainder exceeds a partition, the count up
+// to a tenth below with the shortest last chain is taken.
+inline long capped_partitions(long n, long slots, int b) {
+    auto last_chain = [&](long p) { return (n - (p - 1) * (n / p) + b - 1) / b; };
+    if (slots < 1 || n - slots * (n / slots) <= n / slots) return slots;
+    long best = slots;
+    for (long p = slots - 1; p >= slots - slots / 10; --p)
+        if (last_chain(p) < last_chain(best)) best = p;
+    return best;
+}
