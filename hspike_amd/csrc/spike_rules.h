@@ -1,6 +1,6 @@
-// spike_rules.h -- choices between two kernels that depend on a system's sizes alone (so a system gets the
-// same bits alone and in a batch): plain C++, so that a host compiler builds them too (the tests hold them
-// against measured times of both kernels).
+// spike_rules.h -- choices that depend on a system's sizes and the device alone (so a system gets the same bits
+// alone and in a batch): plain C++, so that a host compiler builds them too (the tests hold them against
+// measured times of both sides).
 #pragma once
 #include <cstdint>
 
@@ -12,7 +12,7 @@
 //   k = 2, 10^6 rows: 1 column 59 / 60, 8 columns 78 / 71, 16 columns 175 / 96
 //   k = 16, 600000 rows, 1 column: 5% fill 36 / 41, 20% 48 / 45; 16 columns: 2% fill 106 / 58
 //   k = 24, 500000 rows, 1 column: 20% fill 48 / 61, 60% 88 / 74; 16 columns: 2% fill 86 / 68
-//   k = 64, 300000 rows: 4% fill (a five-point stencil: 5 entries per row), 16 columns 60 / 71; 64 columns 205 / 182
+//   k = 64, 300000 rows: 2% fill (3.6 entries per row), 16 columns 57 / 69, 64 columns 198 / 182; 5%, 16 columns 63 / 72
 //   k = 64: 8 columns, 20% fill 66 / 81, 35% 110 / 96; 16 columns, 10% 76 / 79, 20% 98 / 85; 32 columns, 10% 135 / 116
 //   k = 128, 200000 rows: 64 columns, 5% fill 201 / 252, 10% 270 / 255, 20% 380 / 280; 32 columns, 20% 202 / 188
 // The lines below are where the two meet over k = 1..128, one-sided and unequal bands, fills of 2% to 100% and
